@@ -141,3 +141,52 @@ def test_dg_image_maps(cuda):
     assert torch.all(img[:, nd3:] == 0)
     np.testing.assert_allclose(img[:, :nd3].cpu().numpy().reshape(-1), (W.cpu().numpy() / 2.5).astype(np.float32))
     assert float(torch.linalg.norm(W2 - W) / torch.linalg.norm(W)) < 1e-7
+
+
+def test_convolution_tiles_agree(cuda):
+    """Every tile of conv3_row_kernel against the smallest one: a batch of 16
+    images of 128^2 runs the four levels on tiles of 512, 256, 128 and 64
+    pixels, one image alone on 64 everywhere.  The tiles add in the same order,
+    so outputs are equal bit for bit; the batch gradient is the mean of the
+    single ones up to the order of its float32 sums (the loss gradient is
+    scaled by 1/16, exactly)."""
+    torch = cuda
+    M, B = 128, 16
+    net, p, x, t, xd, td = _setup(torch, M=M, base=32, in_ld=48, B=B, seed=21)
+    y = torch.empty((B, M, M, net.out_ld), dtype=torch.float32, device="cuda")
+    net.forward(xd, y)
+    loss, g = net.loss_grad(xd, td)
+    one = torch.empty((1, M, M, net.out_ld), dtype=torch.float32, device="cuda")
+    mean, losses = np.zeros(net.n_params), []
+    for k in range(B):
+        net.forward(xd[k:k + 1], one)
+        assert torch.equal(one[0], y[k]), k
+        lk, gk = net.loss_grad(xd[k:k + 1], td[k:k + 1])
+        losses.append(lk)
+        mean += gk.astype(np.float64) / B
+    assert abs(loss - np.mean(losses)) < 1e-6 * loss
+    # float32 partial sums over at most 2^18 pixels in chunks: below 2^-24 * 2^7
+    assert _rel(g, mean) < 1e-5
+
+
+def test_row_convolution_matches_oracle(cuda):
+    """conv3_row_kernel at widths 32 and 16 (conv3_k32_kernel at 8 and 4), with
+    a last slice of 16 input channels, against the oracle."""
+    torch = cuda
+    M, base, B = 32, 32, 1
+    net, p, x, t, xd, td = _setup(torch, M=M, base=base, in_ld=48, B=B, seed=9)
+    y = torch.empty((B, M, M, net.out_ld), dtype=torch.float32, device="cuda")
+    net.forward(xd, y)
+    loss, g = net.loss_grad(xd, td)
+    onet = co.Net(p, net.in_ld, 75, base, emulate_bf16=True)
+    # float32 sums in another order land a few values of every layer on the
+    # other side of a bf16 boundary; fifteen layers of such flips stay below
+    # the effect of all bf16 roundings, which the unrounded network shows
+    ye, y64 = onet.forward(x)[..., :75], co.Net(p, net.in_ld, 75, base).forward(x)[..., :75]
+    noise = _rel(ye, y64)
+    assert noise < 1e-2
+    yg = y.cpu().numpy()[..., :75]
+    assert _rel(yg, ye) < noise and _rel(yg, y64) < 1.2 * noise
+    lo, go = onet.loss_grad(x, t)
+    assert abs(loss - lo) < 1e-3 * lo
+    assert _rel(g, go) < 2e-2

@@ -63,6 +63,14 @@ __device__ __forceinline__ uint16_t f2bf(float f)
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
+// Workgroups are dealt to the 8 XCDs round-robin; give each XCD one contiguous
+// run of work items, so that neighbours share its L2.
+__device__ __forceinline__ int xcd_run(int b, int nblk)
+{
+    const int x = b & 7, q = nblk >> 3, r = nblk & 7;
+    return x * q + (x < r ? x : r) + (b >> 3);
+}
+
 // ------------------------------------------------------------------ conv
 // out[p, co] = act(bias[co] + sum_{tap, ci} in[p + off(tap), ci] w[tap][co][ci])
 // as a GEMM with M = output channels, N = pixels, K = taps x input channels.
@@ -80,7 +88,7 @@ struct ConvArgs {
     int in_ld, in_off, cin;
     int out_ld, out_off, cout;
     int B, H, W, ks, relu;
-    // conv3_k32_kernel with bf16 output: when set, outputs whose value at
+    // conv3_row_kernel and conv3_k32_kernel with bf16 output: when set, outputs whose value at
     // mask[p, mask_off + c] (leading dimension mask_ld) is not positive are
     // stored as 0 (the ReLU backward of the layer below, fused)
     const uint16_t* mask;
@@ -293,32 +301,30 @@ __global__ __launch_bounds__(256) void conv3_tiled_kernel(ConvArgs a)
 // kernel.  A lane l holds channel co + l % 16 and input channels
 // 8 (l / 16) .. + 7 of the weight row; B lane l pixel l % 16 and the same 8
 // input channels; the accumulator layout is that of conv3_tiled_kernel.
-// RT > 1 (images 64 or more pixels wide) makes the tile RT rows of 64 pixels:
-// fewer halo rows per pixel and the slice's weights staged once for RT times
-// the pixels.
-template <int TA, int RT, bool F32OUT>
+// Runs the images less than 16 pixels wide, whose fragments of 16 pixels span
+// rows; conv3_row_kernel takes the wider ones.
+template <int TA, bool F32OUT>
 __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
 {
     constexpr int CO_T = 32 * TA;
-    constexpr int HALO = RT == 1 ? kHaloMax : (RT + 2) * 66;  // halo pixels at most
-    constexpr int NHP = (HALO * 4 + 255) / 256;                // 16-byte halo parts per thread
+    constexpr int NHP = (kHaloMax * 4 + 255) / 256;   // 16-byte halo parts per thread
     constexpr int NWP = (9 * CO_T * 4 + 255) / 256;           // 16-byte weight parts per thread
-    __shared__ __align__(16) uint16_t s_in[HALO * 32];
+    __shared__ __align__(16) uint16_t s_in[kHaloMax * 32];
     __shared__ __align__(16) uint16_t s_w[9 * CO_T * 32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ln = lane & 15, kq = lane >> 4;
-    const int TW = min(a.W, 64), TH = 64 / TW * RT;
+    const int TW = min(a.W, 64), TH = 64 / TW;
     const int tiles_x = a.W / TW, tiles_y = (a.H + TH - 1) / TH;
     const int t = blockIdx.x;
     const int b = t / (tiles_x * tiles_y), ty = (t / tiles_x) % tiles_y, tx = t % tiles_x;
     const int y0 = ty * TH, x0 = tx * TW;
     const int co0 = blockIdx.y * CO_T;
     const int cw = (wave & 1) * (16 * TA);
-    const int pw = (wave >> 1) * 32 * RT;
+    const int pw = (wave >> 1) * 32;
     const int HW2 = TW + 2, NH = (TH + 2) * HW2;
-    int py[2 * RT], px[2 * RT];
+    int py[2], px[2];
 #pragma unroll
-    for (int j = 0; j < 2 * RT; ++j) {
+    for (int j = 0; j < 2; ++j) {
         const int p = pw + 16 * j + ln;
         py[j] = p / TW;
         px[j] = p - py[j] * TW;
@@ -360,11 +366,11 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
             if (woff[k] >= 0 && in_range) wreg[k] = *reinterpret_cast<const uint4*>(a.w + woff[k] + c0);
         }
     };
-    f32x4 acc[TA][2 * RT];
+    f32x4 acc[TA][2];
 #pragma unroll
     for (int i = 0; i < TA; ++i)
 #pragma unroll
-        for (int j = 0; j < 2 * RT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     load(0);
     for (int c0 = 0; c0 < a.cin; c0 += 32) {
@@ -380,19 +386,19 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
 #pragma unroll
         for (int tap = 0; tap < 9; ++tap) {
             const int hy = tap / 3, hx = tap % 3;
-            bf16x8 av[TA], bv[2 * RT];
+            bf16x8 av[TA], bv[2];
 #pragma unroll
             for (int i = 0; i < TA; ++i)
                 av[i] = __builtin_bit_cast(
                     bf16x8, *reinterpret_cast<const uint4*>(s_w + (tap * CO_T + cw + 16 * i + ln) * 32 + 8 * kq));
 #pragma unroll
-            for (int j = 0; j < 2 * RT; ++j)
+            for (int j = 0; j < 2; ++j)
                 bv[j] = __builtin_bit_cast(
                     bf16x8, *reinterpret_cast<const uint4*>(s_in + ((py[j] + hy) * HW2 + px[j] + hx) * 32 + 8 * kq));
 #pragma unroll
             for (int i = 0; i < TA; ++i)
 #pragma unroll
-                for (int j = 0; j < 2 * RT; ++j)
+                for (int j = 0; j < 2; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
         }
     }
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
             bias[0] = b4.x, bias[1] = b4.y, bias[2] = b4.z, bias[3] = b4.w;
         }
 #pragma unroll
-        for (int j = 0; j < 2 * RT; ++j) {
+        for (int j = 0; j < 2; ++j) {
             const int y = y0 + py[j], x = x0 + px[j];
             if (y >= a.H) continue;
             float v[4];
@@ -415,6 +421,158 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
                 if (a.relu) v[q] = fmaxf(v[q], 0.f);
             }
             const size_t pix = (size_t)(b * a.H + y) * a.W + x;
+            const size_t o = pix * a.out_ld + a.out_off + co;
+            if constexpr (F32OUT) {
+                *reinterpret_cast<float4*>(static_cast<float*>(a.out) + o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+                if (a.mask) {
+                    const uint2 mv = *reinterpret_cast<const uint2*>(a.mask + pix * a.mask_ld + a.mask_off + co);
+                    const uint32_t mw[2] = {mv.x, mv.y};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (!(bf2f((uint16_t)(mw[q >> 1] >> (16 * (q & 1)))) > 0.f)) v[q] = 0.f;
+                }
+                const uint32_t lo = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
+                const uint32_t hi = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + o) = make_uint2(lo, hi);
+            }
+        }
+    }
+}
+
+// 3x3 convolution of images at least 16 pixels wide, with the operands of
+// conv3_k32_kernel.  A wave there reads one pixel fragment from LDS per tap
+// for TA MFMAs, and its LDS reads took 1.5-2.3 times the MFMAs' cycles.  Here
+// a wave owns R rows of 16 pixels x 32 output channels and walks the R + 2
+// input rows once per horizontal tap: each fragment it reads feeds the MFMAs
+// of all three vertical taps, so a 32-channel slice costs 18 + 3 (R + 2)
+// fragment reads for 18 R MFMAs.  NW waves cover TW = min(W, 64) x TH pixels;
+// the tile's halo and the slice's weights go from global memory straight to
+// LDS (16 bytes per lane, no registers), halo pixels outside the image and
+// channels past the last from a zero word.  What bounds it now is the latency
+// of one slice's loads and the two or three workgroups a CU holds to cover
+// it.  128^2 x 16 images, forward / backward-data of all 3x3 layers: 270 /
+// 297 us with conv3_k32_kernel at every width, 192 / 192 us here; wider
+// blocks of 64 output channels measured slower at every level (fewer
+// workgroups).
+__device__ uint4 g_zero_part;  // never written
+
+__device__ __forceinline__ void load_to_lds16(const uint16_t* src, uint16_t* lds)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+template <int R, int NW>
+struct RowTile {
+    static constexpr int TA = 2, CO_T = 16 * TA;
+    // halo pixels at most: WX x WY waves, (WY R + 2)(16 WX + 2), WX <= 4
+    static constexpr int halo(int wx) { return (NW / wx * R + 2) * (16 * wx + 2); }
+    static constexpr int HALO = halo(1) > halo(2) ? (halo(1) > halo(4) ? halo(1) : halo(4))
+                                                  : (halo(2) > halo(4) ? halo(2) : halo(4));
+    static constexpr int NHP = (HALO * 4 + 64 * NW - 1) / (64 * NW);      // halo parts per thread
+    static constexpr int NWP = (9 * CO_T * 4 + 64 * NW - 1) / (64 * NW);  // weight parts per thread
+};
+
+template <int R, int NW, bool F32OUT>
+__global__ __launch_bounds__(64 * NW) void conv3_row_kernel(ConvArgs a)
+{
+    using T = RowTile<R, NW>;
+    constexpr int TA = T::TA, CO_T = T::CO_T, NTHR = 64 * NW;
+    // both rounded up to whole rounds of NTHR parts: every lane of a round loads
+    __shared__ __align__(16) uint16_t s_in[T::NHP * NTHR * 8];
+    __shared__ __align__(16) uint16_t s_w[T::NWP * NTHR * 8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ln = lane & 15, kq = lane >> 4, part = tid & 3;
+    const int WX = min(a.W, 64) >> 4, WY = NW / WX;
+    const int TW = 16 * WX, TH = R * WY;
+    const int tiles_x = a.W / TW, tiles_y = a.H / TH;
+    const int ncob = a.cout / CO_T;
+    // consecutive blocks of one XCD share the input tile, then its neighbours
+    const int bid = xcd_run(blockIdx.x, gridDim.x);
+    const int t = bid / ncob, co0 = (bid - t * ncob) * CO_T;
+    const int b = t / (tiles_x * tiles_y), ty = (t / tiles_x) % tiles_y, tx = t % tiles_x;
+    const int y0 = ty * TH, x0 = tx * TW;
+    const int wx = wave % WX, wy = wave / WX;
+    const int HW2 = TW + 2, NH = (TH + 2) * HW2;
+
+    // element offsets of this thread's 16-byte parts (part q = tid + NTHR k:
+    // halo pixel or weight row q / 4, channels 8 (q % 4) ..), -1 for zeros
+    int hoff[T::NHP], woff[T::NWP];
+#pragma unroll
+    for (int k = 0; k < T::NHP; ++k) {
+        const int q = tid + NTHR * k, hp = q >> 2;
+        const int hy = hp / HW2, hx = hp - hy * HW2;
+        const int y = y0 - 1 + hy, x = x0 - 1 + hx;
+        hoff[k] = hp < NH && y >= 0 && y < a.H && x >= 0 && x < a.W
+                      ? ((b * a.H + y) * a.W + x) * a.in_ld + a.in_off + 8 * part
+                      : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < T::NWP; ++k) {
+        const int row = (tid + NTHR * k) >> 2, tap = row / CO_T, co = row - tap * CO_T;
+        woff[k] = tap < 9 ? (tap * a.cout + co0 + co) * a.cin + 8 * part : -1;
+    }
+    const uint16_t* const zero = reinterpret_cast<const uint16_t*>(&g_zero_part);
+    f32x4 acc[TA][R];
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int c0 = 0; c0 < a.cin; c0 += 32) {
+        const bool in_range = c0 + 8 * part < a.cin;  // a last slice of 16 channels is padded with zeros
+        if (c0) __syncthreads();                      // the previous slice is consumed
+#pragma unroll
+        for (int k = 0; k < T::NHP; ++k)
+            load_to_lds16(hoff[k] >= 0 && in_range ? a.in + hoff[k] + c0 : zero, s_in + 8 * (NTHR * k + 64 * wave));
+#pragma unroll
+        for (int k = 0; k < T::NWP; ++k)
+            load_to_lds16(woff[k] >= 0 && in_range ? a.w + woff[k] + c0 : zero, s_w + 8 * (NTHR * k + 64 * wave));
+        __builtin_amdgcn_s_waitcnt(0);  // the loads to LDS have landed
+        __syncthreads();
+#pragma unroll
+        for (int hx = 0; hx < 3; ++hx) {
+            bf16x8 av[3][TA];
+#pragma unroll
+            for (int hy = 0; hy < 3; ++hy)
+#pragma unroll
+                for (int i = 0; i < TA; ++i)
+                    av[hy][i] = __builtin_bit_cast(
+                        bf16x8, *reinterpret_cast<const uint4*>(
+                                    s_w + ((3 * hy + hx) * CO_T + 16 * i + ln) * 32 + 8 * kq));
+            const uint16_t* src = s_in + (wy * R * HW2 + 16 * wx + ln + hx) * 32 + 8 * kq;
+#pragma unroll
+            for (int r = 0; r < R + 2; ++r) {
+                const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + r * HW2 * 32));
+#pragma unroll
+                for (int hy = 0; hy < 3; ++hy) {
+                    if (r - hy < 0 || r - hy >= R) continue;
+#pragma unroll
+                    for (int i = 0; i < TA; ++i)
+                        acc[i][r - hy] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[hy][i], bv, acc[i][r - hy], 0, 0, 0);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TA; ++i) {
+        const int co = co0 + 16 * i + 4 * kq;
+        float bias[4] = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias) {
+            const float4 b4 = *reinterpret_cast<const float4*>(a.bias + co);
+            bias[0] = b4.x, bias[1] = b4.y, bias[2] = b4.z, bias[3] = b4.w;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v[q] = acc[i][r][q] + bias[q];
+                if (a.relu) v[q] = fmaxf(v[q], 0.f);
+            }
+            const size_t pix = (size_t)(b * a.H + y0 + wy * R + r) * a.W + x0 + 16 * wx + ln;
             const size_t o = pix * a.out_ld + a.out_off + co;
             if constexpr (F32OUT) {
                 *reinterpret_cast<float4*>(static_cast<float*>(a.out) + o) = make_float4(v[0], v[1], v[2], v[3]);
@@ -1437,8 +1595,8 @@ int wgrad_tiled_chunks(const Layer& L, int B, int H, int* tiles_per_chunk)
     return (int)((tiles + tpc - 1) / tpc);
 }
 
-// The 3x3 convolutions that run on conv3_k32_kernel (the only one that
-// applies a ReLU-backward mask).
+// The 3x3 convolutions that run on conv3_row_kernel or conv3_k32_kernel (the ones that
+// apply a ReLU-backward mask).
 bool conv_k32_ok(int cin, int cout, int ks, int W, int in_ld, int in_off)
 {
     return ks == 3 && W > 0 && (W & (W - 1)) == 0 && cout % 32 == 0 && cin % 16 == 0 && in_ld % 8 == 0 &&
@@ -1463,21 +1621,43 @@ void launch_conv(const wdg_cnn_s& n, hipStream_t s, const uint16_t* in, int in_l
         const int TA = cout % 64 == 0 ? 2 : 1;
         const dim3 grid((unsigned)tiles, (unsigned)(cout / (32 * TA)));
         if (cin % 32 == 0 || cin > 32) {  // 32-channel slices; a last slice of 16 is zero-padded
-            // taller tiles on images 64 or more pixels wide while about 512 workgroups remain
-            int RT = 1;
-            while (RT < 4 && W >= 64 && H % (2 * RT) == 0 && tiles / (2 * RT) * (cout / (32 * TA)) >= 512) RT *= 2;
-            const dim3 g2((unsigned)(tiles / RT), (unsigned)(cout / (32 * TA)));
-#define WDG_K32_CASE(ta, rt)                                                                       \
-    if (TA == ta && RT == rt) {                                                                    \
-        if (f32out)                                                                                \
-            hipLaunchKernelGGL((conv3_k32_kernel<ta, rt, true>), g2, dim3(256), 0, s, a);          \
-        else                                                                                       \
-            hipLaunchKernelGGL((conv3_k32_kernel<ta, rt, false>), g2, dim3(256), 0, s, a);         \
-        return;                                                                                    \
+            if (W >= 16) {
+                // the largest tile that leaves about two workgroups per CU:
+                // at 128^2 x 16 images 512 pixels per tile on level 0 (32 -> 32
+                // channels 12.7 us, 17.4 us with 256 of four waves), 256, 128
+                // and 64 on levels 1, 2 and 3 (256 -> 256 channels of level 3
+                // 13.5 us, 17.0 us with 256 pixels)
+                const int WX = std::min(W, 64) / 16, cob = cout / 32;
+                auto blocks = [&](int r, int nw) { return (long long)npix / (16 * r * nw) * cob; };
+                auto fits = [&](int r, int nw) { return r * nw / WX <= H && blocks(r, nw) >= 512; };
+#define WDG_ROW_CASE(r, nw)                                                                                     \
+    {                                                                                                           \
+        const dim3 g3((unsigned)blocks(r, nw));                                                                 \
+        if (f32out)                                                                                             \
+            hipLaunchKernelGGL((conv3_row_kernel<r, nw, true>), g3, dim3(64 * nw), 0, s, a);                    \
+        else                                                                                                    \
+            hipLaunchKernelGGL((conv3_row_kernel<r, nw, false>), g3, dim3(64 * nw), 0, s, a);                   \
+        return;                                                                                                 \
     }
-            WDG_K32_CASE(1, 1) WDG_K32_CASE(1, 2) WDG_K32_CASE(1, 4)
-            WDG_K32_CASE(2, 1) WDG_K32_CASE(2, 2) WDG_K32_CASE(2, 4)
-#undef WDG_K32_CASE
+                if (fits(4, 8)) WDG_ROW_CASE(4, 8)
+                if (fits(2, 8)) WDG_ROW_CASE(2, 8)
+                if (fits(2, 4)) WDG_ROW_CASE(2, 4)
+                WDG_ROW_CASE(1, 4)
+#undef WDG_ROW_CASE
+            }
+            // images less than 16 pixels wide
+            if (TA == 2) {
+                if (f32out)
+                    hipLaunchKernelGGL((conv3_k32_kernel<2, true>), grid, dim3(256), 0, s, a);
+                else
+                    hipLaunchKernelGGL((conv3_k32_kernel<2, false>), grid, dim3(256), 0, s, a);
+            } else {
+                if (f32out)
+                    hipLaunchKernelGGL((conv3_k32_kernel<1, true>), grid, dim3(256), 0, s, a);
+                else
+                    hipLaunchKernelGGL((conv3_k32_kernel<1, false>), grid, dim3(256), 0, s, a);
+            }
+            return;
         }
         if (TA == 2) {
             if (f32out)
@@ -1587,7 +1767,7 @@ void relu_grad(wdg_cnn_s& n, hipStream_t s, int level, int C, const float* g1, i
 // Parameter gradients of layer li, then the gradient w.r.t. its pre-ReLU
 // input where that input is act (leading dimension act_ld, offset act_off):
 // the backward-data convolution and the ReLU backward in one pass when
-// conv3_k32_kernel applies (bf16 output masked by act > 0), else the fp32
+// conv_k32_ok holds (bf16 output masked by act > 0), else the fp32
 // input gradient and relu_grad_kernel.  Returns the buffer that holds the
 // result (the other of n.dpre and n.dpre2 than dpre when fused, n.dpre else).
 const uint16_t* bwd_relu(wdg_cnn_s& n, hipStream_t s, int li, const uint16_t* in, int in_ld, int in_off,
