@@ -53,13 +53,8 @@ constexpr int kWaves = 4;     // waves per workgroup of the conv kernels
 constexpr int NLAYER_MAX = 15;  // layers of the network (the Layer enum below)
 constexpr int kChunk = 1024;  // pixels per weight-gradient partial
 
-__device__ __forceinline__ uint16_t f2bf(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// v_cvt_pk_bf16_f32: round to nearest even, infinities kept, NaN quiet
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
@@ -449,43 +444,47 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
 // fragment reads for 18 R MFMAs.  NW waves cover TW = min(W, 64) x TH pixels;
 // the tile's halo and the slice's weights go from global memory straight to
 // LDS (16 bytes per lane, no registers), halo pixels outside the image and
-// channels past the last from a zero word.  What bounds it now is the latency
+// channels past the last read as zeros past
+// the buffer's end.  What bounds it now is the latency
 // of one slice's loads and the two or three workgroups a CU holds to cover
 // it.  128^2 x 16 images, forward / backward-data of all 3x3 layers: 270 /
-// 297 us with conv3_k32_kernel at every width, 192 / 192 us here; wider
-// blocks of 64 output channels measured slower at every level (fewer
-// workgroups).
-__device__ uint4 g_zero_part;  // never written
+// 297 us with conv3_k32_kernel at every width, 182 / 182 us here (192 / 192
+// with per-part pointers and a run-time tile width); blocks of 64 output
+// channels measured slower at every level (fewer workgroups).
+constexpr uint32_t kNoPart = 0xfffffff0u;  // a byte offset past every buffer: such a load gives zeros
 
-__device__ __forceinline__ void load_to_lds16(const uint16_t* src, uint16_t* lds)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes)
 {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);  // raw, 32-bit data
 }
 
-template <int R, int NW>
+// 16 bytes per lane from byte offset voff (per lane) + soff (uniform) of a
+// buffer to consecutive places of LDS (uniform); offsets past the buffer's end give zeros.
+__device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint16_t* lds)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, (int)voff, (int)soff,
+                                             0, 0);
+}
+
+// WX = TW / 16 wave columns
+template <int R, int NW, int WX>
 struct RowTile {
-    static constexpr int TA = 2, CO_T = 16 * TA;
-    // halo pixels at most: WX x WY waves, (WY R + 2)(16 WX + 2), WX <= 4
-    static constexpr int halo(int wx) { return (NW / wx * R + 2) * (16 * wx + 2); }
-    static constexpr int HALO = halo(1) > halo(2) ? (halo(1) > halo(4) ? halo(1) : halo(4))
-                                                  : (halo(2) > halo(4) ? halo(2) : halo(4));
-    static constexpr int NHP = (HALO * 4 + 64 * NW - 1) / (64 * NW);      // halo parts per thread
-    static constexpr int NWP = (9 * CO_T * 4 + 64 * NW - 1) / (64 * NW);  // weight parts per thread
+    static constexpr int TA = 2, CO_T = 16 * TA, NTHR = 64 * NW;
+    static constexpr int TW = 16 * WX, TH = R * (NW / WX), HW2 = TW + 2, NH = (TH + 2) * HW2;
+    static constexpr int NHP = (NH * 4 + NTHR - 1) / NTHR;        // halo parts per thread
+    static constexpr int NWP = (9 * CO_T * 4 + NTHR - 1) / NTHR;  // weight parts per thread
 };
 
-template <int R, int NW, bool F32OUT>
+template <int R, int NW, int WX, bool F32OUT>
 __global__ __launch_bounds__(64 * NW) void conv3_row_kernel(ConvArgs a)
 {
-    using T = RowTile<R, NW>;
-    constexpr int TA = T::TA, CO_T = T::CO_T, NTHR = 64 * NW;
+    using T = RowTile<R, NW, WX>;
+    constexpr int TA = T::TA, CO_T = T::CO_T, NTHR = T::NTHR, TW = T::TW, TH = T::TH, HW2 = T::HW2;
     // both rounded up to whole rounds of NTHR parts: every lane of a round loads
     __shared__ __align__(16) uint16_t s_in[T::NHP * NTHR * 8];
     __shared__ __align__(16) uint16_t s_w[T::NWP * NTHR * 8];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ln = lane & 15, kq = lane >> 4, part = tid & 3;
-    const int WX = min(a.W, 64) >> 4, WY = NW / WX;
-    const int TW = 16 * WX, TH = R * WY;
     const int tiles_x = a.W / TW, tiles_y = a.H / TH;
     const int ncob = a.cout / CO_T;
     // consecutive blocks of one XCD share the input tile, then its neighbours
@@ -494,26 +493,25 @@ __global__ __launch_bounds__(64 * NW) void conv3_row_kernel(ConvArgs a)
     const int b = t / (tiles_x * tiles_y), ty = (t / tiles_x) % tiles_y, tx = t % tiles_x;
     const int y0 = ty * TH, x0 = tx * TW;
     const int wx = wave % WX, wy = wave / WX;
-    const int HW2 = TW + 2, NH = (TH + 2) * HW2;
+    const __amdgpu_buffer_rsrc_t rin = buffer_of(a.in, (uint32_t)(2u * a.B * a.H * a.W * a.in_ld));
+    const __amdgpu_buffer_rsrc_t rw = buffer_of(a.w, (uint32_t)(2u * 9 * a.cout * a.cin));
 
-    // element offsets of this thread's 16-byte parts (part q = tid + NTHR k:
-    // halo pixel or weight row q / 4, channels 8 (q % 4) ..), -1 for zeros
-    int hoff[T::NHP], woff[T::NWP];
+    // byte offsets of this thread's 16-byte parts (part q = tid + NTHR k: halo
+    // pixel or weight row q / 4, channels 8 (q % 4) ..)
+    uint32_t hoff[T::NHP], woff[T::NWP];
 #pragma unroll
     for (int k = 0; k < T::NHP; ++k) {
-        const int q = tid + NTHR * k, hp = q >> 2;
-        const int hy = hp / HW2, hx = hp - hy * HW2;
+        const int hp = (tid + NTHR * k) >> 2, hy = hp / HW2, hx = hp - hy * HW2;
         const int y = y0 - 1 + hy, x = x0 - 1 + hx;
-        hoff[k] = hp < NH && y >= 0 && y < a.H && x >= 0 && x < a.W
-                      ? ((b * a.H + y) * a.W + x) * a.in_ld + a.in_off + 8 * part
-                      : -1;
+        hoff[k] = hp < T::NH && (unsigned)y < (unsigned)a.H && (unsigned)x < (unsigned)a.W
+                      ? 2u * (uint32_t)(((b * a.H + y) * a.W + x) * a.in_ld + a.in_off + 8 * part)
+                      : kNoPart;
     }
 #pragma unroll
     for (int k = 0; k < T::NWP; ++k) {
         const int row = (tid + NTHR * k) >> 2, tap = row / CO_T, co = row - tap * CO_T;
-        woff[k] = tap < 9 ? (tap * a.cout + co0 + co) * a.cin + 8 * part : -1;
+        woff[k] = tap < 9 ? 2u * (uint32_t)((tap * a.cout + co0 + co) * a.cin + 8 * part) : kNoPart;
     }
-    const uint16_t* const zero = reinterpret_cast<const uint16_t*>(&g_zero_part);
     f32x4 acc[TA][R];
 #pragma unroll
     for (int i = 0; i < TA; ++i)
@@ -521,14 +519,17 @@ __global__ __launch_bounds__(64 * NW) void conv3_row_kernel(ConvArgs a)
         for (int r = 0; r < R; ++r) acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (int c0 = 0; c0 < a.cin; c0 += 32) {
-        const bool in_range = c0 + 8 * part < a.cin;  // a last slice of 16 channels is padded with zeros
-        if (c0) __syncthreads();                      // the previous slice is consumed
+        if (c0) __syncthreads();  // the previous slice is consumed
+        if (c0 + 32 > a.cin && c0 + 8 * part >= a.cin) {  // a last slice of 16 channels is padded with zeros
 #pragma unroll
-        for (int k = 0; k < T::NHP; ++k)
-            load_to_lds16(hoff[k] >= 0 && in_range ? a.in + hoff[k] + c0 : zero, s_in + 8 * (NTHR * k + 64 * wave));
+            for (int k = 0; k < T::NHP; ++k) hoff[k] = kNoPart;
 #pragma unroll
-        for (int k = 0; k < T::NWP; ++k)
-            load_to_lds16(woff[k] >= 0 && in_range ? a.w + woff[k] + c0 : zero, s_w + 8 * (NTHR * k + 64 * wave));
+            for (int k = 0; k < T::NWP; ++k) woff[k] = kNoPart;
+        }
+#pragma unroll
+        for (int k = 0; k < T::NHP; ++k) load_to_lds16(rin, hoff[k], 2u * c0, s_in + 8 * (NTHR * k + 64 * wave));
+#pragma unroll
+        for (int k = 0; k < T::NWP; ++k) load_to_lds16(rw, woff[k], 2u * c0, s_w + 8 * (NTHR * k + 64 * wave));
         __builtin_amdgcn_s_waitcnt(0);  // the loads to LDS have landed
         __syncthreads();
 #pragma unroll
@@ -811,6 +812,208 @@ __global__ __launch_bounds__(64 * kWgWaves) void wgrad3_tr_kernel(WgradArgs a)
             for (int r = 0; r < 4; ++r)
                 dst[(size_t)(co0 + 16 * cb + 4 * g + r) * a.cin + ci0 + 16 * ib + ln] = acc[u][cb][r];
     }
+    if (bias) {
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+            float v = bsum[cb];
+            v += __shfl_xor(v, 16);
+            v += __shfl_xor(v, 32);
+            if (g == 0) prow[(size_t)9 * a.cout * a.cin + co0 + 16 * cb + ln] = v;
+        }
+    }
+}
+
+// The same gradients on images at least 16 pixels wide.  wgrad3_tr_kernel reads
+// one fragment of the input from LDS per tap and 32 pixels for two MFMAs, and
+// its workgroups of six waves wrote about 512 partial rows per layer.  Here an
+// MFMA's 32 pixels are one row of 32 (two rows of 16 from two strips on
+// 16-pixel images), and a wave walks the input rows of its RW output rows
+// once: the three horizontally shifted fragments of an input row meet the
+// output gradient rows above, at and below it, so five fragment reads feed 18
+// MFMAs.  Eight waves share a tile of 4 RW rows: wave w owns input-channel
+// block w % 2 and output rows RW (w / 2) .., both output-channel blocks, all
+// nine taps (72 accumulator registers); the four row groups are added in LDS
+// in fixed order at the end, so a layer writes at most 256 partial rows.  The
+// next tile's loads go straight to the other LDS buffer during this tile's
+// MFMAs, their offsets found once and their borders by one test of a bit mask
+// (with the addresses recomputed per tile the kernel was bound by that integer
+// arithmetic: 302 us against 261 for all layers).  128^2 x 16 images, weight
+// gradients and reductions of all 3x3 layers: 422 us with wgrad3_tr_kernel,
+// 337 here.  What bounds it now is the latency of a tile's loads with one tile
+// in flight per CU.
+constexpr int kWgRowTarget = 256;  // workgroups a layer aims for: one per CU
+
+// TW = 32, or 16 on 16-pixel images (two strips per tile)
+template <int RW, int TW>
+struct WgRow {
+    static constexpr int NT = 512, TH = 4 * RW, SUB = 32 / TW;
+    static constexpr int PX = 32 * TH;                                   // pixels of a tile
+    static constexpr int HW2 = TW + 2, NH1 = (TH + 2) * HW2;             // halo pixels of a strip
+    static constexpr int NXP = (SUB * NH1 * 4 + NT - 1) / NT, NDP = PX * 4 / NT;  // 16-byte parts per thread
+    static constexpr int x_elems = SUB * NH1 * 32, d_elems = PX * 32;
+    static constexpr size_t bytes = 2 * (size_t)(x_elems + d_elems) * sizeof(uint16_t);
+};
+
+template <int RW, int TW>
+__global__ __launch_bounds__(512) void wgrad3_row_kernel(WgradArgs a)
+{
+    using T = WgRow<RW, TW>;
+    constexpr int TH = T::TH, NT = T::NT, SUB = T::SUB, HW2 = T::HW2, NH1 = T::NH1;
+    __shared__ __align__(16) uint16_t smem[T::bytes / sizeof(uint16_t)];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int g = lane >> 4, ln = lane & 15, la = ln & 3, lj = ln >> 2;
+    const int strips_x = a.W / TW, strips_y = a.H / TH;  // powers of two
+    const int nstrips = a.B * strips_y * strips_x;
+    const int ntiles = (nstrips + SUB - 1) / SUB;
+    const int shx = __builtin_ctz((unsigned)strips_x), shy = __builtin_ctz((unsigned)strips_y);
+    // the workgroups of one chunk (every pair of channel blocks) are neighbours
+    // on one XCD, so its pixels come from that L2 once
+    const int ncob = a.cout / 32, npair = ncob * ((a.cin + 31) / 32);
+    const int bid = xcd_run(blockIdx.x, gridDim.x), chunk = bid / npair, pair = bid - chunk * npair;
+    const int co0 = (pair % ncob) * 32, ci0 = (pair / ncob) * 32;
+    const int t0 = chunk * a.tiles_per_chunk, t1 = min(ntiles, t0 + a.tiles_per_chunk);
+    const int ib = wave & 1, rg = wave >> 1;
+    const bool bias = ib == 0 && ci0 == 0;
+    const __amdgpu_buffer_rsrc_t rx = buffer_of(a.in, (uint32_t)(2u * a.B * a.H * a.W * a.in_ld));
+    const __amdgpu_buffer_rsrc_t rd = buffer_of(a.dout, (uint32_t)(2u * a.B * a.H * a.W * a.dout_ld));
+    f32x4 acc[9][2];
+#pragma unroll
+    for (int u = 0; u < 9; ++u) acc[u][0] = acc[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum[2] = {0.f, 0.f};
+    // The tile's 16-byte parts: halo pixel q / 4 of the tile's strips in turn,
+    // then output-gradient pixel q / 4 ([row][32 pixels], strips side by side).
+    // Found once: each part's byte offset from its strip's first pixel, and on
+    // which borders of the strip's halo it lies (bits top, bottom, left, right).
+    const int part = tid & 3;
+    const bool ci_in = ci0 + 8 * part < a.cin;
+    int xoff[T::NXP], doff[T::NDP];
+    uint32_t border[T::NXP];
+#pragma unroll
+    for (int k = 0; k < T::NXP; ++k) {
+        const int hp = (tid + NT * k) >> 2, h = hp >= NH1 ? hp - NH1 : hp, hy = h / HW2, hx = h - hy * HW2;
+        xoff[k] = 2 * (((hy - 1) * a.W + hx - 1) * a.in_ld + a.in_off + ci0 + 8 * part);
+        border[k] = (hy == 0 ? 1u : 0u) | (hy == TH + 1 ? 2u : 0u) | (hx == 0 ? 4u : 0u) | (hx == TW + 1 ? 8u : 0u) |
+                    (ci_in ? 0u : 16u);
+    }
+#pragma unroll
+    for (int k = 0; k < T::NDP; ++k) {
+        const int pp = (tid + NT * k) >> 2, c = pp & (TW - 1);
+        doff[k] = 2 * (((pp >> 5) * a.W + c) * a.dout_ld + co0 + 8 * part);
+    }
+    auto load = [&](int t, uint16_t* sx, uint16_t* sd) {
+        int first[SUB];       // the strips' first pixels
+        uint32_t outside[SUB];  // the halo borders outside the image; no such strip: everything
+#pragma unroll
+        for (int st = 0; st < SUB; ++st) {
+            const int sid = t * SUB + st;
+            const int b = sid >> (shx + shy), sy = (sid >> shx) & (strips_y - 1), sc = sid & (strips_x - 1);
+            first[st] = (b * a.H + sy * TH) * a.W + sc * TW;
+            outside[st] = sid < nstrips ? 16u | (sy == 0 ? 1u : 0u) | (sy == strips_y - 1 ? 2u : 0u) |
+                                              (sc == 0 ? 4u : 0u) | (sc == strips_x - 1 ? 8u : 0u)
+                                        : 32u;
+        }
+#pragma unroll
+        for (int k = 0; k < T::NXP; ++k) {
+            const int hp = (tid + NT * k) >> 2;
+            const bool second = SUB == 2 && hp >= NH1;
+            const uint32_t out = second ? outside[SUB - 1] : outside[0];
+            const int f = second ? first[SUB - 1] : first[0];
+            if (hp < SUB * NH1)
+                load_to_lds16(rx, (border[k] & out) || (SUB == 2 && out == 32u) ? kNoPart : (uint32_t)xoff[k] + 2u * (uint32_t)f * (uint32_t)a.in_ld,
+                              0, sx + 8 * (NT * k + 64 * wave));
+        }
+#pragma unroll
+        for (int k = 0; k < T::NDP; ++k) {
+            const bool second = SUB == 2 && (((tid + NT * k) >> 2) & 31) >= TW;
+            const uint32_t out = second ? outside[SUB - 1] : outside[0];
+            const int f = second ? first[SUB - 1] : first[0];
+            load_to_lds16(rd, SUB == 2 && out == 32u ? kNoPart : (uint32_t)doff[k] + 2u * (uint32_t)f * (uint32_t)a.dout_ld, 0,
+                          sd + 8 * (NT * k + 64 * wave));
+        }
+    };
+    constexpr int kBuf = T::x_elems + T::d_elems;
+    if (t0 < t1) load(t0, smem, smem + T::x_elems);
+    // this lane's pixels of a row: 8 g + lj and 8 g + lj + 4, in strip 8 g / TW
+    const int px = 8 * g + lj, pst = 8 * g >= TW ? 1 : 0;
+    const int hbase = pst * NH1 + px - pst * TW + rg * RW * HW2;
+    for (int t = t0; t < t1; ++t) {
+        __builtin_amdgcn_s_waitcnt(0);  // this tile's loads to LDS have landed
+        __syncthreads();                // and the other buffer is consumed
+        const int cur = ((t - t0) & 1) * kBuf, nxt = kBuf - cur;
+        if (t + 1 < t1) load(t + 1, smem + nxt, smem + nxt + T::x_elems);
+        const uint16_t* const sd = smem + cur + T::x_elems + (rg * RW * 32 + px) * 32 + 4 * la;
+        const uint16_t* const sx = smem + cur + hbase * 32 + 16 * ib + 4 * la;
+        bf16x8 A[3][2];  // output-gradient rows r - 2, r - 1, r of this wave, by row % 3
+#pragma unroll
+        for (int r = 0; r < RW + 2; ++r) {
+            if (r < RW) {
+                const uint16_t* p = sd + r * 32 * 32;
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) A[r % 3][cb] = lds_tr_pair(p + 16 * cb, p + 4 * 32 + 16 * cb);
+                if (bias) {
+#pragma unroll
+                    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) bsum[cb] += (float)A[r % 3][cb][q];
+                }
+            }
+#pragma unroll
+            for (int hx = 0; hx < 3; ++hx) {
+                const uint16_t* p = sx + (r * HW2 + hx) * 32;
+                const bf16x8 bv = lds_tr_pair(p, p + 4 * 32);
+#pragma unroll
+                for (int hy = 0; hy < 3; ++hy) {
+                    const int o = r - hy;  // halo row r is the tap hy input of output row r - hy
+                    if (o < 0 || o >= RW) continue;
+#pragma unroll
+                    for (int cb = 0; cb < 2; ++cb)
+                        acc[3 * hy + hx][cb] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[o % 3][cb], bv, acc[3 * hy + hx][cb], 0, 0, 0);
+                }
+            }
+        }
+    }
+    // add the four row groups in order: groups 1, 2, 3 leave their sums in LDS
+    // one after another ([ib][18 x 4 values][lane], bias sums after them)
+    float* const red = reinterpret_cast<float*>(smem) + ib * 74 * 64;
+    for (int k = 1; k < 4; ++k) {
+        __syncthreads();
+        if (rg == k) {
+#pragma unroll
+            for (int u = 0; u < 9; ++u)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) red[(u * 8 + cb * 4 + r) * 64 + lane] = acc[u][cb][r];
+            red[72 * 64 + lane] = bsum[0];
+            red[73 * 64 + lane] = bsum[1];
+        }
+        __syncthreads();
+        if (rg == 0) {
+#pragma unroll
+            for (int u = 0; u < 9; ++u)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[u][cb][r] += red[(u * 8 + cb * 4 + r) * 64 + lane];
+            bsum[0] += red[72 * 64 + lane];
+            bsum[1] += red[73 * 64 + lane];
+        }
+    }
+    if (rg != 0) return;  // no barriers below
+    // accumulator lane l: co = co0 + 16 cb + 4 (l / 16) + r, ci = ci0 + 16 ib + l % 16
+    const size_t row = (size_t)9 * a.cout * a.cin + a.cout;
+    float* const prow = a.partial + (size_t)chunk * row;
+    if (ci0 + 16 * ib < a.cin)  // a last block of 16 input channels is padded with zeros
+#pragma unroll
+        for (int u = 0; u < 9; ++u) {
+            float* dst = prow + (size_t)u * a.cout * a.cin;
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    dst[(size_t)(co0 + 16 * cb + 4 * g + r) * a.cin + ci0 + 16 * ib + ln] = acc[u][cb][r];
+        }
     if (bias) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
@@ -1617,6 +1820,28 @@ int wgrad1_chunks(int B, int H, int* tiles_per_chunk)
     return (int)((tiles + tpc - 1) / tpc);
 }
 
+// wgrad3_row_kernel's output rows per wave: the taller tile while it leaves a
+// workgroup per CU.
+int wgrad_row_rw(const Layer& L, int B, int H)
+{
+    const long long pairs = (long long)(L.cout / 32) * ((L.cin + 31) / 32);
+    return (long long)B * H * H / 512 * pairs >= kWgRowTarget ? 4 : 2;
+}
+
+// Tiles per chunk of wgrad3_row_kernel: as many chunks as give at most
+// kWgRowTarget workgroups (two more than the CUs would run as a second round
+// of the whole launch).  Returns the chunk count.
+int wgrad_row_chunks(const Layer& L, int B, int H, int* tiles_per_chunk)
+{
+    const int rw = wgrad_row_rw(L, B, H), px = 128 * rw;
+    const long long tiles = ((long long)B * H * H + px - 1) / px;
+    const long long pairs = std::max<long long>(1, (long long)(L.cout / 32) * ((L.cin + 31) / 32));
+    const long long most = std::max<long long>(1, kWgRowTarget / pairs);
+    const int tpc = (int)((tiles + most - 1) / most);
+    if (tiles_per_chunk) *tiles_per_chunk = tpc;
+    return (int)((tiles + tpc - 1) / tpc);
+}
+
 // Tiles per chunk of the transposing-load weight gradient: enough chunks for about kWgTarget
 // workgroups, at most 16 tiles each.  Returns the chunk count.
 int wgrad_tiled_chunks(const Layer& L, int B, int H, int* tiles_per_chunk)
@@ -1635,6 +1860,17 @@ bool conv_k32_ok(int cin, int cout, int ks, int W, int in_ld, int in_off)
 {
     return ks == 3 && W > 0 && (W & (W - 1)) == 0 && cout % 32 == 0 && cin % 16 == 0 && in_ld % 8 == 0 &&
            in_off % 8 == 0 && (cin % 32 == 0 || cin > 32);
+}
+
+template <int R, int NW, int WX>
+void launch_conv_row(hipStream_t s, const ConvArgs& a, bool f32out)
+{
+    using T = RowTile<R, NW, WX>;
+    const dim3 grid((unsigned)((long long)a.B * (a.H / T::TH) * (a.W / T::TW) * (a.cout / T::CO_T))), block(T::NTHR);
+    if (f32out)
+        hipLaunchKernelGGL((conv3_row_kernel<R, NW, WX, true>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((conv3_row_kernel<R, NW, WX, false>), grid, block, 0, s, a);
 }
 
 void launch_conv(const wdg_cnn_s& n, hipStream_t s, const uint16_t* in, int in_ld, int in_off, int cin,
@@ -1666,11 +1902,12 @@ void launch_conv(const wdg_cnn_s& n, hipStream_t s, const uint16_t* in, int in_l
                 auto fits = [&](int r, int nw) { return r * nw / WX <= H && blocks(r, nw) >= 512; };
 #define WDG_ROW_CASE(r, nw)                                                                                     \
     {                                                                                                           \
-        const dim3 g3((unsigned)blocks(r, nw));                                                                 \
-        if (f32out)                                                                                             \
-            hipLaunchKernelGGL((conv3_row_kernel<r, nw, true>), g3, dim3(64 * nw), 0, s, a);                    \
+        if (WX == 4)                                                                                            \
+            launch_conv_row<r, nw, 4>(s, a, f32out);                                                            \
+        else if (WX == 2)                                                                                       \
+            launch_conv_row<r, nw, 2>(s, a, f32out);                                                            \
         else                                                                                                    \
-            hipLaunchKernelGGL((conv3_row_kernel<r, nw, false>), g3, dim3(64 * nw), 0, s, a);                   \
+            launch_conv_row<r, nw, 1>(s, a, f32out);                                                            \
         return;                                                                                                 \
     }
                 if (fits(4, 8)) WDG_ROW_CASE(4, 8)
@@ -1755,9 +1992,24 @@ void bwd(wdg_cnn_s& n, hipStream_t s, int li, const uint16_t* in, int in_ld, int
     const long long nw = (long long)ntap * L.cout * L.cin;
     WgradArgs wa{in, dpre, n.partial, in_ld, in_off, L.cin, L.cout, L.cout, B, H, H, L.ks, 1};
     if (wgrad_tr_ok(L, H, in_ld, in_off)) {
-        const int wchunks = wgrad_tiled_chunks(L, B, H, &wa.tiles_per_chunk);
-        hipLaunchKernelGGL(wgrad3_tr_kernel, dim3(wchunks, L.cout / 32, (L.cin + 31) / 32), dim3(64 * kWgWaves), 0, s,
-                           wa);
+        int wchunks;
+        if (H >= 16) {
+            wchunks = wgrad_row_chunks(L, B, H, &wa.tiles_per_chunk);
+            const dim3 grid((unsigned)(wchunks * (L.cout / 32) * ((L.cin + 31) / 32)));
+            const bool tall = wgrad_row_rw(L, B, H) == 4, wide = H >= 32;
+            if (tall && wide)
+                hipLaunchKernelGGL((wgrad3_row_kernel<4, 32>), grid, dim3(512), 0, s, wa);
+            else if (tall)
+                hipLaunchKernelGGL((wgrad3_row_kernel<4, 16>), grid, dim3(512), 0, s, wa);
+            else if (wide)
+                hipLaunchKernelGGL((wgrad3_row_kernel<2, 32>), grid, dim3(512), 0, s, wa);
+            else
+                hipLaunchKernelGGL((wgrad3_row_kernel<2, 16>), grid, dim3(512), 0, s, wa);
+        } else {
+            wchunks = wgrad_tiled_chunks(L, B, H, &wa.tiles_per_chunk);
+            hipLaunchKernelGGL(wgrad3_tr_kernel, dim3(wchunks, L.cout / 32, (L.cin + 31) / 32), dim3(64 * kWgWaves), 0,
+                               s, wa);
+        }
         // rows of [weights][bias]: the bias follows the weights in the parameter vector
         reduce_chunks(s, n.partial, nw + L.cout, wchunks, n.g + L.w);
         if (gin)
@@ -2051,7 +2303,9 @@ int wdg_hip_cnn_create(int M, int in_ld, int out_channels, int base_width, int m
             const int H = M >> L.level;
             // the largest chunk count any batch size up to max_batch uses
             long long tchunks = 0;
-            for (int bb = 1; bb <= max_batch; ++bb) tchunks = std::max<long long>(tchunks, wgrad_tiled_chunks(L, bb, H, nullptr));
+            for (int bb = 1; bb <= max_batch; ++bb)
+                tchunks = std::max<long long>({tchunks, wgrad_tiled_chunks(L, bb, H, nullptr),
+                                               wgrad_row_chunks(L, bb, H, nullptr)});
             const long long chunks =
                 std::max<long long>(((long long)max_batch * H * H + kChunk - 1) / kChunk, tchunks);
             const long long bchunks = ((long long)max_batch * H * H + kBiasChunk - 1) / kBiasChunk;
