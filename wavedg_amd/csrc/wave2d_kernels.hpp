@@ -639,12 +639,13 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
     // FP64 stage outputs with streaming stores at orders whose elements do not
     // fill whole wavefronts: the workgroup's elements are one contiguous block
     // per array, staged in the workgroup's state tile and stored as 16-byte
-    // pieces (EPB 3 n^2 a multiple of the values per piece keeps every
-    // workgroup block 16-byte aligned).  Every thread of the workgroup takes
-    // part in its barriers.
+    // pieces where EPB 3 n^2 is even, which keeps every workgroup block 16-byte
+    // aligned, and as single values where it is odd (n = 7 and 9; still whole
+    // lines per wavefront: 400^2 P = 6 stage 179 -> 153 us, 384^2 P = 8 269 ->
+    // 231 us against strided stores).  Every thread of the workgroup takes part in its barriers.
     constexpr int VPR = 16 / (int)sizeof(R);  // values per 16-byte piece
-    constexpr bool WG_BLOCKS = NT && !F32 && N != 8 && (OUT == M_OUT_STAGE0 || OUT == M_OUT_STAGE) &&
-                               (Shape<N, TGT>::EPB * 3 * N * N) % VPR == 0;
+    constexpr int VPP = (Shape<N, TGT>::EPB * 3 * N * N) % VPR == 0 ? VPR : 1;  // values per staged piece
+    constexpr bool WG_BLOCKS = NT && !F32 && N != 8 && (OUT == M_OUT_STAGE0 || OUT == M_OUT_STAGE);
     if constexpr (!WG_BLOCKS) {
         if (!active) return;
     }
@@ -712,7 +713,7 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
                     const piece_t* t2 = reinterpret_cast<const piece_t*>(tile);
                     piece_t* d2 = reinterpret_cast<piece_t*>(dst);
 #pragma unroll
-                    for (int k = lane; k < PIECES; k += 64) __builtin_nontemporal_store(t2[k], d2 + k);
+                    for (int k = lane; k < PIECES; k += 64) st_stream<NT>(d2 + k, t2[k]);
                     __builtin_amdgcn_wave_barrier();
                 };
                 const size_t eb = gb + (size_t)el * 3 * L::NN;  // the element's first value
@@ -729,12 +730,13 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
                         tile[g + 2] = v2;
                     }
                     __syncthreads();
-                    const piece_t* t2 = reinterpret_cast<const piece_t*>(tile);
-                    piece_t* d2 = reinterpret_cast<piece_t*>(dst);
-                    const int npc = nval / VPR;
-                    for (int k = threadIdx.x; k < npc; k += blockDim.x) __builtin_nontemporal_store(t2[k], d2 + k);
-                    for (int k = npc * VPR + threadIdx.x; k < nval; k += blockDim.x)
-                        __builtin_nontemporal_store(tile[k], dst + k);
+                    typedef typename std::conditional<VPP == 1, R, piece_t>::type staged_t;
+                    const staged_t* t2 = reinterpret_cast<const staged_t*>(tile);
+                    staged_t* d2 = reinterpret_cast<staged_t*>(dst);
+                    const int npc = nval / VPP;
+                    for (int k = threadIdx.x; k < npc; k += blockDim.x) st_stream<NT>(d2 + k, t2[k]);
+                    if constexpr (VPP > 1)
+                        for (int k = npc * VPP + threadIdx.x; k < nval; k += blockDim.x) st_stream<NT>(dst + k, tile[k]);
                     __syncthreads();
                 };
                 store_block(static_cast<R*>(a.du) + gb, d0, d1, d2);
