@@ -177,3 +177,43 @@ def test_exact_mass_any_n_var(cuda, nvar):
     torch.cuda.synchronize()
     assert rel_l2(y.cpu().numpy(), ow.mass_action(x, nvar=nvar)) < 1e-13
     assert rel_l2(z.cpu().numpy(), ow.mass_inv(x, nvar=nvar)) < 1e-12
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("leg", [False, True])
+def test_exact_fused_rhs_every_order(cuda, n, leg):
+    """The fused right-hand side (on the Gauss points; collocated for a
+    Gauss-Legendre basis) with forcing at every order, the last workgroup
+    partly filled, mixed boundary codes, against the oracle's quadrature."""
+    torch = cuda
+    v, e = mesh_case("skewed6x5")
+    om, gm = O.Mesh(v, e), capi.Mesh(v, e)
+    bc = bc_codes(gm.n_boundary, "mixed")
+    ow = O.Wave(om, n, bc, approx_quad=False, legendre=leg)
+    gw = capi.Wave2D(gm, n, bc, approx_quad=False, basis=capi.GAUSS_LEGENDRE if leg else capi.GAUSS_LOBATTO)
+    u, F = random_state(gw.ndof, 5 + n), random_state(gw.ndof, 50 + n)
+    y = torch.zeros(gw.ndof, dtype=torch.float64, device="cuda")
+    gw.rhs(_dev(torch, u), y, _dev(torch, F), 0.7)
+    torch.cuda.synchronize()
+    assert rel_l2(y.cpu().numpy(), ow.rhs(u, F, 0.7)) < TOL
+
+
+def test_exact_streaming_stage(cuda):
+    """The fused stage with non-temporal stores (stage arrays above the 256
+    MiB cache) equals the ordinary one on a part of the mesh that its steps
+    cannot tell apart: two meshes whose left columns are the same."""
+    torch = cuda
+    n, ny = 5, 64
+    out = []
+    for nx in (2400, 200):
+        mesh = capi.Mesh.uniform_rect(nx, 0.0, nx / 64.0, ny, 0.0, 1.0)
+        gw = capi.Wave2D(mesh, n, np.zeros(mesh.n_boundary, dtype=np.int32), approx_quad=False)
+        assert (3 * gw.ndof * 8 > 256 << 20) == (nx == 2400)
+        u = torch.zeros((ny, nx, n * n * 3), dtype=torch.float64, device="cuda")
+        g = torch.Generator(device="cuda").manual_seed(3)
+        u[:, :200] = torch.randn((ny, 200, n * n * 3), dtype=torch.float64, device="cuda", generator=g)
+        u = u.reshape(-1)
+        gw.rk4(u, 0.5 / 64 / n**2, 2)  # ten stages: nothing right of column 190 is compared
+        torch.cuda.synchronize()
+        out.append(u.reshape(ny, nx, -1)[:, :150].clone())
+    assert rel_l2(out[0].cpu().numpy(), out[1].cpu().numpy()) < TOL

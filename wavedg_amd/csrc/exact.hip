@@ -358,83 +358,104 @@ __global__ __launch_bounds__(kBlk) void exact_mass_kernel(const KArgs a, const d
 }
 
 // ---------------------------------------------------------------- fused stage
-// The whole right-hand side / RK stage for the default rules (QV = N volume,
-// QE = N + 1 edge points) in one kernel.  E elements share an NT-lane
-// workgroup.  In every tensor pass a lane owns one (element, variable, line),
-// keeps the line in registers and reads the 1D tables as uniform operands
-// through the scalar cache (row-contiguous copies).  Two LDS regions per
-// element carry the transposes between passes:
-//   RA: u -> u at the volume points -> edge-point traces -> t1 -> M^{-1} r
-//   RB: xi-interpolated u -> Df, then Pg -> staged traces -> edge fluxes and
-//       their projections -> t3
-// The operator output r stays in the registers of the lane that owns its
-// line from the volume pass to the mass matrix; the face projections are
-// added there.  Arrays read along a line of lanes have odd strides in
-// doubles (the L* pitches), so a wave's reads spread over the LDS banks.
+// The whole right-hand side / RK stage for the default rules on a
+// Gauss-Lobatto basis in one kernel.  Every integral of the operator is of a
+// polynomial that the N-point Gauss-Legendre rule integrates exactly as well:
+// det J and the metric terms of a bilinear map are affine, so the volume and
+// mass integrands have degree at most 2N - 1 per direction, and so have the
+// edge fluxes on straight sides.  The same operator is therefore collocated
+// on the Gauss points: u is interpolated there (values
+// uh(i, j) at x_i, x_j), the contravariant fluxes and the derivative matrix
+// DG of the Gauss basis act point by point and line by line, the mass matrix
+// is the diagonal w_i w_j det J(i, j), and the result is interpolated back to
+// the nodes, du/dt = B(x)B uh_t.  That is 6 N^3 multiplications per variable
+// (two interpolations each way and one derivative per direction) where volume
+// rule, edge rule and fast diagonalisation took 14 N^3, and 8 barriers
+// instead of 15.  On a Gauss-Legendre basis the nodes are the points, so
+// those handles run the collocated kernels (apply_op).
+//
+// E elements share an NT-lane workgroup.  In every tensor pass a lane owns one
+// (element, variable, line), keeps the line in registers and reads the 1D
+// tables as uniform operands through the scalar cache (row-contiguous
+// copies).  LDS regions per element:
+//   RA: u -> uh -> eta-interpolated result     RB: xi-interpolated u -> xi
+//   derivative -> du/dt   TR: neighbour traces -> edge fluxes
+// Arrays read along a line of lanes have odd strides in doubles (the L*
+// pitches), so a wave's reads spread over the LDS banks.  What bounds it: the
+// LDS is busy 56 % of the time, vector issue 46 %, in passes that the 3-4
+// waves per SIMD its tiles allow do not fully overlap.  Per stage, before and
+// now: 330 x 335 P = 5 129 -> 107 us, 512^2 P = 7 483 -> 415 us (1.551 GB,
+// 3.7 TB/s), 256^2 P = 6 95 -> 73 us.
 template <int N>
 struct StageShape {
     static constexpr int cmax(int x, int y) { return x > y ? x : y; }
     static constexpr int odd(int x) { return x | 1; }
-    static constexpr int QV = N, QE = N + 1, NN = N * N;
+    static constexpr int NN = N * N;
     static constexpr int NT = (N == 6 || N == 8) ? 128 : 64;  // fills the lanes best
     static constexpr int E = NT / (3 * N);                     // 3N line lanes per element
-    static constexpr int LS = odd(3 * N);    // (3, N, N) arrays: d + 3 i + LS j
-    static constexpr int LQ = odd(3 * QV);   // u at the volume points: d + 3 i + LQ j
-    static constexpr int LP = odd(N);        // xi-interpolated u: (d + 3 i) LP + l
-    static constexpr int LD = odd(QV);       // Df or Pg: (d + 3 k) LD + j
-    static constexpr int LT = odd(N);        // staged side traces: row LT
-    static constexpr int LE = odd(QE);       // edge-point traces and fluxes: row LE
-    static constexpr int SA = cmax(cmax(LS * N, LQ * QV), 24 * LE);
-    static constexpr int SB = cmax(cmax(3 * QV * LP, 3 * N * LD), cmax(cmax(24 * LT, 12 * LE + 12 * N), LS * N));
-    static constexpr int S = SA + SB;
+    static constexpr int LS = odd(3 * N);  // (3, N, N) arrays: d + 3 i + LS j
+    static constexpr int LP = odd(N);      // transposed ones: (d + 3 i) LP + j
+    static constexpr int SA = LS * N;
+    static constexpr int SB = cmax(3 * N * LP, LS * N);
+    static constexpr int ST = 12 * LP;     // rows (3 s + d) LP
+    static constexpr int S = SA + SB + ST;
 };
 
 // out_o = sum_k T[o NK + k] x[k] for o = 0 .. NO - 1, with T a uniform
-// table read through the scalar cache.  The row of output o + 1 is requested
-// while output o is computed; the compiler barrier keeps later rows from all
-// being hoisted to the top, which would exhaust the scalar registers.
+// table read through the scalar cache.  Rows come in pairs, the next pair
+// requested while this one is used (scalar loads return out of order, so every
+// wait is for all of them; pairs halve the waits: 112 -> 110 us at 330 x 335
+// P = 5); the compiler barrier keeps later rows from all being hoisted to the
+// top, which would exhaust the scalar registers.
 template <int NO, int NK, typename Store>
 __device__ __forceinline__ void contract_rows(const double* __restrict__ T, const double (&x)[NK], Store store)
 {
-    double r[2][NK];
+    constexpr int RB = 2, NB = (NO + RB - 1) / RB;  // rows per batch, batches
+    double r[2][RB][NK];
 #pragma unroll
-    for (int k = 0; k < NK; ++k) r[0][k] = T[k];
+    for (int q = 0; q < RB; ++q)
 #pragma unroll
-    for (int o = 0; o < NO; ++o) {
-        if (o + 1 < NO) {
+        for (int k = 0; k < NK; ++k) r[0][q][k] = T[q * NK + k];
 #pragma unroll
-            for (int k = 0; k < NK; ++k) r[(o + 1) % 2][k] = T[(o + 1) * NK + k];
-        }
-        double acc = 0.0;
+    for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int k = 0; k < NK; ++k) acc += r[o % 2][k] * x[k];
-        store(o, acc);
+        for (int q = 0; q < RB; ++q)
+            if ((b + 1) * RB + q < NO) {
+#pragma unroll
+                for (int k = 0; k < NK; ++k) r[(b + 1) % 2][q][k] = T[((b + 1) * RB + q) * NK + k];
+            }
+#pragma unroll
+        for (int q = 0; q < RB; ++q)
+            if (b * RB + q < NO) {
+                double acc = 0.0;
+#pragma unroll
+                for (int k = 0; k < NK; ++k) acc += r[b % 2][q][k] * x[k];
+                store(b * RB + q, acc);
+            }
         asm volatile("" ::: "memory");
     }
 }
 
-// At n = 8 on the Gauss-Lobatto basis the kernel fits 96 VGPRs without
-// spilling, so it asks for 5 waves per SIMD instead of the 4 that its
-// natural 97 allow (the LDS tiles allow 4.5 on average).
-template <int N, bool LEG>
-__global__ __launch_bounds__(StageShape<N>::NT, (N == 8 && !LEG) ? 5 : 1) void exact_stage_kernel(
-    const KArgs a, const double* __restrict__ tab, int kid)
+// FORCE: the load vector is added; NTS: outputs as non-temporal stores
+// (KArgs::nt_store; contiguous runs of 8-byte values per wavefront).
+template <int N, bool FORCE, bool NTS>
+__global__ __launch_bounds__(StageShape<N>::NT) void exact_stage_kernel(const KArgs a, const double* __restrict__ tab,
+                                                                        int kid)
 {
     using Sh = StageShape<N>;
-    constexpr int QV = Sh::QV, QE = Sh::QE, NN = Sh::NN, E = Sh::E, NT = Sh::NT;
-    constexpr int LS = Sh::LS, LQ = Sh::LQ, LP = Sh::LP, LD = Sh::LD, LT = Sh::LT, LE = Sh::LE;
+    constexpr int NN = Sh::NN, E = Sh::E, NT = Sh::NT, LS = Sh::LS, LP = Sh::LP;
     constexpr int NS = (E * 3 * NN + NT - 1) / NT;  // state values per lane
-    static_assert(QV == N, "the line lanes of the volume passes assume QV == N");
+    constexpr int NF = (E * 4 * N + NT - 1) / NT;   // face points per lane
     __shared__ double s_mem[E * Sh::S];
     __shared__ double s_geo[E * 6];
     // the epilogue's scalars, parked in LDS so that they hold no scalar
     // registers through the passes (which would spill them)
     __shared__ double s_par[4];
     __shared__ double* s_ptr[3];
-    // each XCD walks one contiguous run of elements, so neighbour traces and
-    // the block's own side traces are read through the L2 that loaded them
+    // each XCD walks one contiguous run of elements, so neighbour traces are
+    // read through the L2 that loaded the neighbour
     const int lane = threadIdx.x, e0 = xcd_block(blockIdx.x, gridDim.x) * E, nel = a.nel;
-    const int mode = kModeOf[kid];
+    const int mode = kModeOf[kid], out = mode & M_OUTMASK;
     if (lane == 0) {
         s_par[0] = a.rk_a;
         s_par[1] = a.rk_b;
@@ -447,7 +468,7 @@ __global__ __launch_bounds__(StageShape<N>::NT, (N == 8 && !LEG) ? 5 : 1) void e
     const double* __restrict__ u = static_cast<const double*>(a.u_in);
     auto RA = [&](int e) { return s_mem + e * Sh::S; };
     auto RB = [&](int e) { return s_mem + e * Sh::S + Sh::SA; };
-    auto sidx = [](int d, int i, int j) { return d + 3 * i + LS * j; };
+    auto TR = [&](int e) { return s_mem + e * Sh::S + Sh::SA + Sh::SB; };
     const int nvalid = nel - e0 < E ? nel - e0 : E;
     // line lanes: element le, variable ld, line lk
     const int le = lane / (3 * N), lj = lane % (3 * N), ld = lj % 3, lk = lj / 3;
@@ -456,266 +477,256 @@ __global__ __launch_bounds__(StageShape<N>::NT, (N == 8 && !LEG) ? 5 : 1) void e
     // the block's elements are contiguous in HBM: every load is issued before
     // the first wait
     const double* ublk = u + (size_t)e0 * 3 * NN;
+    const int cnt = nvalid * 3 * NN;
     double v[NS];
+    int off[NS];  // the places of this lane's values in the LDS regions (clamped past the last)
 #pragma unroll
     for (int r = 0; r < NS; ++r) {
-        const int it = lane + r * NT;
-        v[r] = it < nvalid * 3 * NN ? ublk[it] : 0.0;
+        const int it = min(lane + r * NT, cnt - 1), e = it / (3 * NN), k = it - e * (3 * NN);
+        v[r] = ublk[it];
+        off[r] = e * Sh::S + k + (LS - 3 * N) * (k / (3 * N));
     }
     const double gv = lane < nvalid * 6 ? a.geom[6 * (size_t)e0 + lane] : 0.0;
+    // this lane's face points: element, side, place along it; neighbour trace
+    // base and flags (points past the last repeat it, which changes nothing)
+    int fe[NF], fs[NF], fk[NF], fx[NF], fy[NF];
+    double tr[NF][3];
 #pragma unroll
-    for (int r = 0; r < NS; ++r) {
-        const int it = lane + r * NT, e = it / (3 * NN), k = it % (3 * NN);
-        if (it < nvalid * 3 * NN) RA(e)[k + (LS - 3 * N) * (k / (3 * N))] = v[r];
+    for (int r = 0; r < NF; ++r) {
+        const int it = min(lane + r * NT, nvalid * 4 * N - 1), q4 = it / N;
+        fe[r] = q4 >> 2;
+        fs[r] = q4 & 3;
+        fk[r] = it - q4 * N;
+        const FaceNb f = a.fnb[4 * (size_t)e0 + q4];
+        fx[r] = f.x;
+        fy[r] = f.y;
+        tr[r][0] = tr[r][1] = tr[r][2] = 0.0;
+        if (f.x >= 0) {
+            const double* q = u + (f.x + fk[r] * (f.y >> 16));
+            tr[r][0] = q[0];
+            tr[r][1] = q[1];
+            tr[r][2] = q[2];
+        }
     }
+    double Rf[FORCE ? N : 1];
+    if constexpr (FORCE) {
+        // the load vector on the Gauss basis, (B'(x)B') F: along xi by lane
+        // (d, j), along eta by lane (d, i)
+        if (lon) {
+            const double* F = static_cast<const double*>(a.force) + (size_t)(e0 + le) * 3 * NN + ld + 3 * N * lk;
+            double x[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) x[k] = F[3 * k];
+            double* W = RB(le);
+            contract_rows<N, N>(tab + kTabBL, x, [&](int i, double acc) { W[(ld + 3 * i) * LP + lk] = acc; });
+        }
+        __syncthreads();
+        if (lon) {
+            const double* W = RB(le) + (ld + 3 * lk) * LP;
+            double x[N];
+#pragma unroll
+            for (int l = 0; l < N; ++l) x[l] = W[l];
+            contract_rows<N, N>(tab + kTabBL, x, [&](int l, double acc) { Rf[l] = acc; });
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < NS; ++r) s_mem[off[r]] = v[r];
     if (lane < nvalid * 6) s_geo[lane] = gv;
+#pragma unroll
+    for (int r = 0; r < NF; ++r) {
+        double* T = TR(fe[r]) + 3 * fs[r] * LP + fk[r];
+        T[0] = tr[r][0];
+        T[LP] = tr[r][1];
+        T[2 * LP] = tr[r][2];
+    }
     __syncthreads();
-    // ---- volume: the passes of div_2d_q (Div.cpp:469-588)
+    // ---- interpolation to the Gauss points
     // PU(l, d, i) = sum_k P(i, k) u(d, k, l)          lane (d, l)
     if (lon) {
         double x[N];
 #pragma unroll
-        for (int k = 0; k < N; ++k) x[k] = RA(le)[sidx(ld, k, lk)];
+        for (int k = 0; k < N; ++k) x[k] = RA(le)[ld + 3 * k + LS * lk];
         double* PU = RB(le);
-        contract_rows<QV, N>(tab + kTabPVT, x, [&](int i, double acc) { PU[(ld + 3 * i) * LP + lk] = acc; });
+        contract_rows<N, N>(tab + kTabPVT, x, [&](int i, double acc) { PU[(ld + 3 * i) * LP + lk] = acc; });
+    }
+    // the neighbour traces, each row in place by one lane
+    for (int it = lane; it < nvalid * 12; it += NT) {
+        double* T = TR(it / 12) + LP * (it % 12);
+        double x[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) x[k] = T[k];
+        contract_rows<N, N>(tab + kTabPVT, x, [&](int q, double acc) { T[q] = acc; });
     }
     __syncthreads();
-    // UQ(d, i, j) = sum_l P(j, l) PU(l, d, i)          lane (d, i)
+    // uh(d, i, j) = sum_l P(j, l) PU(l, d, i)          lane (d, i)
     if (lon) {
         const double* PU = RB(le) + (ld + 3 * lk) * LP;
         double x[N];
 #pragma unroll
         for (int l = 0; l < N; ++l) x[l] = PU[l];
         double* UQ = RA(le);
-        contract_rows<QV, N>(tab + kTabPVT, x, [&](int jq, double acc) { UQ[ld + 3 * lk + LQ * jq] = acc; });
+        contract_rows<N, N>(tab + kTabPVT, x, [&](int jq, double acc) { UQ[ld + 3 * lk + LS * jq] = acc; });
     }
     __syncthreads();
-    // contravariant fluxes of f = (u, p, 0), g = (v, 0, p) at the points, then
-    //   Df(j, d, k) = sum_i D(i, k) F(d, i, j)   (lane (d, j)),  r  = sum_j P(j, l) Df(j, d, k)
-    //   Pg(j, d, k) = sum_i P(i, k) G(d, i, j),                  r += sum_j D(j, l) Pg(j, d, k)
-    // with r(d, k, :) in the registers of lane (d, k)
-    double R[N];
+    // The fluxes f = (u, p, 0), g = (v, 0, p) of variable d are m1 U1 and
+    // m2 U2 with U1, U2 the variables at offsets o1, o2 and m1, m2 zero or one,
+    // so a lane folds them into its element's map coefficients once.
+    const double m1 = ld == 2 ? 0.0 : 1.0, m2 = ld == 1 ? 0.0 : 1.0;
+    const int o1 = ld == 0 ? 1 : 0, o2 = ld == 0 ? 2 : 0;
+    // ---- xi derivative, DP(k, d, j) = sum_i w_i DG(i, k) F(d, i, j): lane (d, j),
+    // F = w_j (y_eta f - x_eta g)
+    if (lon) {
+        const double* g = s_geo + 6 * le;
+        const double wj = tab[kTabWV + lk];
+        const double c1 = wj * m1 * g[3], h1 = wj * m1 * g[5], c2 = -(wj * m2) * g[2], h2 = -(wj * m2) * g[4];
+        const double* UQ = RA(le) + LS * lk;
+        double acc[N];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        if (lon) {
-            const int jq = lk;
-            const double* g = s_geo + 6 * le;
-            const double ax = g[0], ay = g[1], cx = g[2], cy = g[3], hx = g[4], hy = g[5];
-            const double eta = tab[kTabXV + jq], wj = tab[kTabWV + jq];
-            const double* UQ = RA(le) + LQ * jq;
-            double acc[N];
-#pragma unroll
-            for (int k = 0; k < N; ++k) acc[k] = 0.0;
+        for (int k = 0; k < N; ++k) acc[k] = 0.0;
 #pragma unroll 2
-            for (int i = 0; i < QV; ++i) {
-                const double xi = tab[kTabXV + i], W = tab[kTabWV + i] * wj;
-                const double p = UQ[3 * i], uu = UQ[3 * i + 1], vv = UQ[3 * i + 2];
-                const double s1 = ld == 0 ? uu : (ld == 1 ? p : 0.0);
-                const double s2 = ld == 0 ? vv : (ld == 2 ? p : 0.0);
-                double f;
-                if (half == 0) {
-                    const double X_eta = (cx + hx * xi) * W, Y_eta = (cy + hy * xi) * W;
-                    f = Y_eta * s1 - X_eta * s2;
-                } else {
-                    const double X_xi = (ax + hx * eta) * W, Y_xi = (ay + hy * eta) * W;
-                    f = -Y_xi * s1 + X_xi * s2;
-                }
+        for (int i = 0; i < N; ++i) {
+            const double xi = tab[kTabXV + i];
+            const double f = fma(h1, xi, c1) * UQ[3 * i + o1] + fma(h2, xi, c2) * UQ[3 * i + o2];
 #pragma unroll
-                for (int k = 0; k < N; ++k) acc[k] += tab[(half == 0 ? kTabDVT : kTabPVT) + k + N * i] * f;
-            }
-            double* DP = RB(le);
-#pragma unroll
-            for (int k = 0; k < N; ++k) DP[(ld + 3 * k) * LD + jq] = acc[k];
+            for (int k = 0; k < N; ++k) acc[k] += tab[kTabDGT + k + N * i] * f;
         }
-        __syncthreads();
-        if (lon) {
-            const double* DP = RB(le) + (ld + 3 * lk) * LD;
-            double x[QV];
+        double* DP = RB(le);
 #pragma unroll
-            for (int jq = 0; jq < QV; ++jq) x[jq] = DP[jq];
-            contract_rows<N, QV>(tab + (half == 0 ? kTabPV : kTabDV), x, [&](int l, double acc) {
-                if (half == 0)
-                    R[l] = acc;
-                else
-                    R[l] += acc;
-            });
-        }
-        __syncthreads();
+        for (int k = 0; k < N; ++k) DP[(ld + 3 * k) * LP + lk] = acc[k];
     }
-    // ---- faces (EdgeFlux<false>): own and exterior traces at the side's nodes
-    {
-        constexpr int NF = (E * 4 * N + NT - 1) / NT;
-        int nb[NF], inf[NF];
+    // ---- edge fluxes at the Gauss points of the sides: the own trace by the
+    // face interpolation PG(m) = phi_m(-1) of the Gauss basis, closed form of
+    // EdgeFlux for the wave equation, weighted by w ds
 #pragma unroll
-        for (int r = 0; r < NF; ++r) {
-            const int it = lane + r * NT, e = it / (4 * N), s = (it % (4 * N)) / N;
-            const bool ok = it < nvalid * 4 * N;
-            nb[r] = ok ? a.nbr[4 * (size_t)(e0 + e) + s] : -1;
-            inf[r] = ok ? a.info[4 * (size_t)(e0 + e) + s] : 0;
-        }
-        double tr[NF][6];
-#pragma unroll
-        for (int r = 0; r < NF; ++r) {
-            const int it = lane + r * NT, e = it / (4 * N), j = it % (4 * N), s = j / N, k = j % N;
-            if (it >= nvalid * 4 * N) continue;
-            side_trace<N>(u + ((size_t)(e0 + e) * NN + side_node<N>(s, k)) * 3, s, LEG, tab + kTabPF, tr[r][0],
-                          tr[r][1], tr[r][2]);
-            if (nb[r] >= 0) {
-                const int kk = ((inf[r] >> 2) & 1) ? (N - 1 - k) : k;
-                side_trace<N>(u + ((size_t)nb[r] * NN + side_node<N>(inf[r] & 3, kk)) * 3, inf[r] & 3, LEG,
-                              tab + kTabPF, tr[r][3], tr[r][4], tr[r][5]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < NF; ++r) {
-            const int it = lane + r * NT, e = it / (4 * N), j = it % (4 * N), s = j / N, k = j % N;
-            if (it >= nvalid * 4 * N) continue;
-            if (nb[r] < 0) {
-                double n0, n1, ds;
-                side_normal(s_geo + 6 * e, s, n0, n1, ds);
-                boundary_state((inf[r] >> 8) & 0xff, n0, n1, tr[r][0], tr[r][1], tr[r][2], tr[r][3], tr[r][4],
-                               tr[r][5]);
-            }
-            double* T = RB(e) + 6 * LT * s + k;  // rows: own p, u, v, exterior p, u, v
-#pragma unroll
-            for (int c = 0; c < 6; ++c) T[c * LT] = tr[r][c];
-        }
-    }
-    __syncthreads();
-    // traces at the edge points
-    for (int it = lane; it < E * 24; it += NT) {
-        const int e = it / 24, j = it % 24;  // row j = 6 s + 3 (own | exterior) + d
-        if (e >= nvalid) continue;
-        const double* T = RB(e) + LT * j;
-        double x[N];
-#pragma unroll
-        for (int k = 0; k < N; ++k) x[k] = T[k];
-        double* Q = RA(e) + LE * j;
-        contract_rows<QE, N>(tab + kTabPET, x, [&](int q, double acc) { Q[q] = acc; });
-    }
-    __syncthreads();
-    // closed-form flux at every edge point, weighted by w ds
-    for (int it = lane; it < E * 4 * QE; it += NT) {
-        const int e = it / (4 * QE), j = it % (4 * QE), s = j / QE, q = j % QE;
-        if (e >= nvalid) continue;
+    for (int r = 0; r < NF; ++r) {
+        if (lane + r * NT >= nvalid * 4 * N) continue;  // the flux replaces the trace: once
+        const int e = fe[r], s = fs[r], k = fk[r];
         double n0, n1, ds;
-        side_normal(s_geo + 6 * e, s, n0, n1, ds);
-        const double* Q = RA(e) + 6 * LE * s + q;
-        const double A0 = Q[0 * LE], A1 = Q[1 * LE], A2 = Q[2 * LE];
-        const double B0 = Q[3 * LE], B1 = Q[4 * LE], B2 = Q[5 * LE];
-        const double wds = tab[kTabWE + q] * ds;
-        double* Cf = RB(e) + 3 * LE * s + q;
-        Cf[0 * LE] = wds * (a.ha * (n0 * (A1 + B1) + n1 * (A2 + B2)) + a.hb * (A0 - B0));
-        const double cf = wds * (a.ha * (A0 + B0) + a.hb * (n0 * (A1 - B1) + n1 * (A2 - B2)));
-        Cf[1 * LE] = n0 * cf;
-        Cf[2 * LE] = n1 * cf;
-    }
-    __syncthreads();
-    // projection onto each side's nodes: FP(s, d, k)
-    for (int it = lane; it < E * 12; it += NT) {
-        const int e = it / 12, j = it % 12;  // j = 3 s + d
-        if (e >= nvalid) continue;
-        const double* Cf = RB(e) + LE * j;
-        double c[QE];
-#pragma unroll
-        for (int q = 0; q < QE; ++q) c[q] = Cf[q];
-        double* FP = RB(e) + 12 * LE + N * j;
-        contract_rows<N, QE>(tab + kTabPE, c, [&](int k, double val) { FP[k] = val; });
-    }
-    __syncthreads();
-    // ---- M^{-1} (r + s F) by fast diagonalisation
-    // lane (d, i): r(d, i, :) += faces and forcing; t1(d, i, b) = sum_j V(j, b) r(d, i, j)
-    if (lon) {
-        if (mode & M_FORCE) {
-            const double* F = static_cast<const double*>(a.force) + (size_t)(e0 + le) * 3 * NN + ld + 3 * lk;
-#pragma unroll
-            for (int l = 0; l < N; ++l) R[l] += F[3 * N * l] * a.fs;
+        {
+            // as side_normal, with the length's reciprocal by Newton steps
+            const double* g = s_geo + 6 * e;
+            const double sh = (s == 0 || s == 3) ? -1.0 : 1.0;
+            const double dx = 2.0 * ((s & 1) ? g[2] + sh * g[4] : g[0] + sh * g[4]);
+            const double dy = 2.0 * ((s & 1) ? g[3] + sh * g[5] : g[1] + sh * g[5]);
+            const double l2 = dx * dx + dy * dy, il = rsqrt_nr(l2), sil = s >= 2 ? -il : il;
+            n0 = dy * sil;
+            n1 = -dx * sil;
+            ds = 0.5 * (l2 * il);
         }
-        const double* FP = RB(le) + 12 * LE + N * ld;  // side s at + 3 N s
-        if constexpr (LEG) {
-            // node (i, l) is row l of side 0, row N-1-i of side 1, row N-1-l
-            // of side 2 and row i of side 3 (legendre_transpose_2d,
-            // FaceProlongator.cpp:908-934)
-            const double* Pf = tab + kTabPF;
-            const double f0 = FP[0 * 3 * N + lk], f2 = FP[2 * 3 * N + lk];
-            const double p1 = Pf[N - 1 - lk], p3 = Pf[lk];
+        // first point of the line through side point k and its step inwards
+        const int first = s == 0 ? 3 * k : s == 1 ? 3 * (N - 1) + LS * k : s == 2 ? 3 * k + LS * (N - 1) : LS * k;
+        const int step = s == 0 ? LS : s == 1 ? -3 : s == 2 ? -LS : 3;
+        const double* q = RA(e) + first;
+        double A0 = 0.0, A1 = 0.0, A2 = 0.0;
 #pragma unroll
-            for (int l = 0; l < N; ++l)
-                R[l] += Pf[l] * f0 + Pf[N - 1 - l] * f2 + p1 * FP[1 * 3 * N + l] + p3 * FP[3 * 3 * N + l];
+        for (int m = 0; m < N; ++m) {
+            const double w = tab[kTabPG + m];
+            A0 = fma(w, q[m * step + 0], A0);
+            A1 = fma(w, q[m * step + 1], A1);
+            A2 = fma(w, q[m * step + 2], A2);
+        }
+        double* C = TR(e) + 3 * s * LP + k;  // the flux takes the trace's place
+        double B0, B1, B2;
+        if (fx[r] >= 0) {
+            B0 = C[0];
+            B1 = C[LP];
+            B2 = C[2 * LP];
         } else {
-            R[0] += FP[0 * 3 * N + lk];
-            R[N - 1] += FP[2 * 3 * N + lk];
-            if (lk == N - 1) {
-#pragma unroll
-                for (int l = 0; l < N; ++l) R[l] += FP[1 * 3 * N + l];
-            }
-            if (lk == 0) {
-#pragma unroll
-                for (int l = 0; l < N; ++l) R[l] += FP[3 * 3 * N + l];
-            }
+            boundary_state((fy[r] >> 8) & 0xff, n0, n1, A0, A1, A2, B0, B1, B2);
         }
-        double* T1 = RA(le);
-        contract_rows<N, N>(tab + kTabV, R, [&](int b, double t) { T1[sidx(ld, lk, b)] = t; });
+        const double wds = tab[kTabWV + k] * ds;
+        C[0] = wds * (a.ha * (n0 * (A1 + B1) + n1 * (A2 + B2)) + a.hb * (A0 - B0));
+        const double cf = wds * (a.ha * (A0 + B0) + a.hb * (n0 * (A1 - B1) + n1 * (A2 - B2)));
+        C[LP] = n0 * cf;
+        C[2 * LP] = n1 * cf;
     }
     __syncthreads();
-    // lane (d, b): t2(d, a, b) = sum_i V(i, a) t1(d, i, b) / (d0 + d1 lam_a + d2 lam_b),
-    //              t3(d, i, b) = sum_a V(i, a) t2(d, a, b)
+    // ---- lane (d, i): eta derivative of G = w_i (-y_xi f + x_xi g), the xi
+    // derivative, the faces lifted along their lines with PG (point (i, l) is
+    // row l of side 0, row N-1-i of side 1, row N-1-l of side 2 and row i of
+    // side 3), the diagonal mass matrix w_i w_l det J (w_l is in the table), and
+    // the way back along eta, t(d, i, j) = sum_l B(j, l) / w_l (w_l uh_t(d, i, l))
+    double T1[N];
     if (lon) {
-        double x[N];
+        const double* g = s_geo + 6 * le;
+        const double wi = tab[kTabWV + lk];
+        const double c1 = -(wi * m1) * g[1], h1 = -(wi * m1) * g[5], c2 = wi * m2 * g[0], h2 = wi * m2 * g[4];
+        const double* UQ = RA(le) + 3 * lk;
+        const double* DP = RB(le) + (ld + 3 * lk) * LP;
+        double R[N];
 #pragma unroll
-        for (int i = 0; i < N; ++i) x[i] = RA(le)[sidx(ld, i, lk)];
+        for (int l = 0; l < N; ++l) R[l] = DP[l];
+#pragma unroll 2
+        for (int j = 0; j < N; ++j) {
+            const double eta = tab[kTabXV + j];
+            const double* U = UQ + LS * j;
+            const double f = fma(h1, eta, c1) * U[o1] + fma(h2, eta, c2) * U[o2];
+#pragma unroll
+            for (int l = 0; l < N; ++l) R[l] += tab[kTabDGT + l + N * j] * f;
+        }
+        const double* C = TR(le) + LP * ld;  // side s at + 3 LP s
+        const double* PG = tab + kTabPG;
+        const double f0 = C[lk], f2 = C[2 * 3 * LP + lk];
+        const double p1 = PG[N - 1 - lk], p3 = PG[lk];
         double d0, d1, d2;
-        detj_affine(s_geo + 6 * le, d0, d1, d2);
-        const double db = d0 + d2 * tab[kTabLam + lk];
-        double t2[N];
-        contract_rows<N, N>(tab + kTabV, x, [&](int aa, double t) { t2[aa] = t * recip(db + d1 * tab[kTabLam + aa]); });
-        double* T3 = RB(le);
-        contract_rows<N, N>(tab + kTabVT, t2, [&](int i, double t) { T3[sidx(ld, i, lk)] = t; });
-    }
-    __syncthreads();
-    // lane (d, i): y(d, i, j) = sum_b V(j, b) t3(d, i, b)
-    if (lon) {
-        double x[N];
+        detj_affine(g, d0, d1, d2);
+        const double di = wi * (d0 + d1 * tab[kTabXV + lk]), de = wi * d2;
 #pragma unroll
-        for (int b = 0; b < N; ++b) x[b] = RB(le)[sidx(ld, lk, b)];
-        double* Y = RA(le);
-        contract_rows<N, N>(tab + kTabVT, x, [&](int j, double t) { Y[sidx(ld, lk, j)] = t; });
+        for (int l = 0; l < N; ++l) {
+            double x = R[l] + (PG[l] * f0 + PG[N - 1 - l] * f2 + p1 * C[1 * 3 * LP + l] + p3 * C[3 * 3 * LP + l]);
+            if constexpr (FORCE) x += Rf[l] * a.fs;
+            R[l] = x * recip(di + de * tab[kTabXV + l]);
+        }
+        contract_rows<N, N>(tab + kTabBWT, R, [&](int j, double t) { T1[j] = t; });
+    }
+    __syncthreads();  // uh is consumed
+    if (lon) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) RA(le)[ld + 3 * lk + LS * j] = T1[j];
     }
     __syncthreads();
-    // ---- epilogue: right-hand side, or the RK stage (and WaveHoltz accumulation)
-    const int out = mode & M_OUTMASK;
+    // the epilogue's loads, in flight through the last pass
     const size_t gb = (size_t)e0 * 3 * NN;
     const volatile double* vpar = s_par;
     double* const volatile* vptr = s_ptr;
     double* const uo = vptr[0] + gb;
-    if (out == M_OUT_RHS) {
-#pragma unroll
-        for (int r = 0; r < NS; ++r) {
-            const int it = lane + r * NT, e = it / (3 * NN), k = it % (3 * NN);
-            if (it < nvalid * 3 * NN) uo[it] = RA(e)[k + (LS - 3 * N) * (k / (3 * N))];
-        }
-        return;
-    }
-    const double rk_a = vpar[0], rk_b = vpar[1], dt = vpar[2], ac = vpar[3];
     double* const du = vptr[1] + gb;
     double* const acc = vptr[2] + gb;
     double dv[NS], av[NS];
 #pragma unroll
     for (int r = 0; r < NS; ++r) {
-        const int it = lane + r * NT;
-        const bool ok = it < nvalid * 3 * NN;
-        dv[r] = ok && out != M_OUT_STAGE0 ? du[it] : 0.0;
-        av[r] = ok && (mode & M_ACC) ? acc[it] : 0.0;
+        const int it = min(lane + r * NT, cnt - 1);
+        dv[r] = out == M_OUT_STAGE ? du[it] : 0.0;
+        av[r] = (mode & M_ACC) ? acc[it] : 0.0;
     }
+    // lane (d, j): du/dt(d, i, j) = sum_k B(i, k) t(d, k, j)
+    if (lon) {
+        double x[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) x[k] = RA(le)[ld + 3 * k + LS * lk];
+        double* Y = RB(le);
+        contract_rows<N, N>(tab + kTabBLT, x, [&](int i, double t) { Y[ld + 3 * i + LS * lk] = t; });
+    }
+    __syncthreads();
+    // ---- epilogue: right-hand side, or the RK stage (and WaveHoltz accumulation)
+    if (out == M_OUT_RHS) {
+#pragma unroll
+        for (int r = 0; r < NS; ++r) {
+            const int it = lane + r * NT;
+            if (it < cnt) uo[it] = s_mem[off[r] + Sh::SA];
+        }
+        return;
+    }
+    const double rk_a = vpar[0], rk_b = vpar[1], dt = vpar[2], ac = vpar[3];
 #pragma unroll
     for (int r = 0; r < NS; ++r) {
-        const int it = lane + r * NT, e = it / (3 * NN), k = it % (3 * NN);
-        if (it >= nvalid * 3 * NN) continue;
-        const double rhs = RA(e)[k + (LS - 3 * N) * (k / (3 * N))];
+        const int it = lane + r * NT;
+        if (it >= cnt) continue;
+        const double rhs = s_mem[off[r] + Sh::SA];
         const double dd = (out == M_OUT_STAGE0 ? 0.0 : rk_a * dv[r]) + dt * rhs;
-        du[it] = dd;
+        st_stream<NTS>(du + it, dd);
         const double w = v[r] + rk_b * dd;
-        uo[it] = w;
+        st_stream<NTS>(uo + it, w);
         if (mode & M_ACC) acc[it] = av[r] + ac * w;
     }
 }
@@ -724,12 +735,16 @@ template <int N>
 void launch_stage(int kid, const KArgs& a, const double* tab, hipStream_t s)
 {
     constexpr int E = StageShape<N>::E;
-    if (a.leg)
-        hipLaunchKernelGGL((exact_stage_kernel<N, true>), dim3((a.nel + E - 1) / E), dim3(StageShape<N>::NT), 0, s, a,
-                           tab, kid);
+    const dim3 grid((a.nel + E - 1) / E), block(StageShape<N>::NT);
+    const bool force = (kModeOf[kid] & M_FORCE) != 0;
+    if (force && a.nt_store)
+        hipLaunchKernelGGL((exact_stage_kernel<N, true, true>), grid, block, 0, s, a, tab, kid);
+    else if (force)
+        hipLaunchKernelGGL((exact_stage_kernel<N, true, false>), grid, block, 0, s, a, tab, kid);
+    else if (a.nt_store)
+        hipLaunchKernelGGL((exact_stage_kernel<N, false, true>), grid, block, 0, s, a, tab, kid);
     else
-        hipLaunchKernelGGL((exact_stage_kernel<N, false>), dim3((a.nel + E - 1) / E), dim3(StageShape<N>::NT), 0, s,
-                           a, tab, kid);
+        hipLaunchKernelGGL((exact_stage_kernel<N, false, false>), grid, block, 0, s, a, tab, kid);
 }
 
 template <int N>

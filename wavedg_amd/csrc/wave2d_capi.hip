@@ -295,6 +295,14 @@ void apply_op(wdg_wave2d op, int kid, const KArgs& a, hipStream_t s)
         wdg::launch_exact_face(op->n, a, t, 1, 0, s);
     } else if (kid == wdg::K_BC) {
         wdg::launch_exact_face(op->n, a, t, 0, 1, s);
+    } else if (op->exact_fused() && op->leg) {
+        // The nodes of a Gauss-Legendre basis are the points of the default
+        // volume rule, and every integrand of the operator has a degree that
+        // this rule integrates exactly (also on the edges, where the default
+        // rule has one point more): the exact operator is the collocated one
+        // (200^2 P = 5: 56 us per stage with the general kernel, 30 us here).
+        launch_wave(op->n, kid, 0, op->sched, a, s);
+        return;
     } else if (op->exact_fused()) {
         wdg::launch_exact_stage(op->n, kid, a, op->d_extab, s);
     } else {
@@ -979,11 +987,21 @@ static int create_exact(wdg_mesh mesh, int n_colloc, int basis_type, const int* 
             for (int c = 0; c < cols; ++c)
                 for (int r = 0; r < rows; ++r) tab[dst + c + cols * r] = tab[src + r + rows * c];
         };
-        transpose(wdg::kTabPV, nq_volume, n, wdg::kTabPVT);
-        transpose(wdg::kTabDV, nq_volume, n, wdg::kTabDVT);
-        transpose(wdg::kTabPE, nq_edge, n, wdg::kTabPET);
-        transpose(wdg::kTabV, n, n, wdg::kTabVT);
         const double xm1 = -1.0;
+        if (nq_volume == n) {  // the Gauss basis of the fused stage kernel
+            const double* xv = tab.data() + wdg::kTabXV;
+            transpose(wdg::kTabPV, n, n, wdg::kTabPVT);
+            wdg::lagrange_derivative_matrix(n, xv, n, xv, tab.data() + wdg::kTabBL);
+            transpose(wdg::kTabBL, n, n, wdg::kTabDGT);
+            const double* wv = tab.data() + wdg::kTabWV;
+            for (int i = 0; i < n; ++i)
+                for (int k = 0; k < n; ++k) tab[wdg::kTabDGT + k + n * i] *= wv[i];
+            wdg::lagrange_interpolation_matrix(n, xv, n, op->x.data(), tab.data() + wdg::kTabBL);
+            transpose(wdg::kTabBL, n, n, wdg::kTabBLT);
+            for (int j = 0; j < n; ++j)
+                for (int l = 0; l < n; ++l) tab[wdg::kTabBWT + l + n * j] = tab[wdg::kTabBLT + l + n * j] / wv[l];
+            wdg::lagrange_interpolation_matrix(n, xv, 1, &xm1, tab.data() + wdg::kTabPG);
+        }
         wdg::lagrange_interpolation_matrix(n, op->x.data(), 1, &xm1, tab.data() + wdg::kTabPF);
         op->exact = true;
         op->nqv = nq_volume;

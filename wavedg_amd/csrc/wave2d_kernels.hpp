@@ -905,10 +905,12 @@ bool rtc_edgeflux(RtcFlux* f, const double* u, double* out, const double* corner
 // Exact-quadrature operators, FP64 (exact.hip).  Tables are device arrays,
 // column-major (n_quad, n): P(q, k) = phi_k(x_q), D(q, k) = phi_k'(x_q).
 // One table block per handle, offsets in doubles: volume rule x, w, P, D;
-// edge rule x, w, P; mass matrices A, B, V, lam (ExactMassTables); and the
-// transposes of P, D (volume), P (edge) and V, row-major copies whose rows
-// are contiguous for the fused stage kernel's scalar loads; and the face
-// interpolation weights of a Gauss-Legendre basis.
+// edge rule x, w, P; mass matrices A, B, V, lam (ExactMassTables); and for the
+// fused stage kernel (default rules), which works on the Gauss basis of the
+// volume rule's points, with rows contiguous for its scalar loads: the
+// transpose of P (points by nodes), the transposed derivative matrix DG of
+// the Gauss basis times the point weights, its values B at the nodes and their transpose, and its
+// face interpolation weights.
 enum : int {
     kTabXV = 0,
     kTabWV = 10,
@@ -922,11 +924,13 @@ enum : int {
     kTabV = 540,
     kTabLam = 640,
     kTabPVT = 650,
-    kTabDVT = 750,
-    kTabPET = 850,
-    kTabVT = 950,
+    kTabDGT = 750,
+    kTabBL = 850,
+    kTabBLT = 950,
     kTabPF = 1050,  // phi_k(-1): face interpolation of a Gauss-Legendre basis
-    kTabSize = 1060,
+    kTabPG = 1060,  // the same of the Gauss basis
+    kTabBWT = 1070,  // BLT with column l divided by the volume weight w_l
+    kTabSize = 1170,
 };
 struct ExactTables {
     const double* xv;  // volume rule (Div<false>)
@@ -954,7 +958,8 @@ void launch_exact_face(int n, const KArgs& a, const ExactTables& t, int interior
 void launch_exact_mass(int n, const KArgs& a, const double* r, const ExactMassTables& m, int kid, hipStream_t s,
                        int nv = 3);
 // The whole RHS / RK stage (kid >= K_RHS) for the default rules (n volume
-// points, n + 1 edge points) in one kernel; tab is the handle's table block.
+// points, n + 1 edge points) on a Gauss-Lobatto basis in one kernel; tab is
+// the handle's table block.
 void launch_exact_stage(int n, int kid, const KArgs& a, const double* tab, hipStream_t s);
 
 // Host-side launchers, one translation unit per N (wave2d_kernels_n.hip).
