@@ -138,3 +138,28 @@ def test_solve_many_batches_small_problems_and_solves_large_ones_alone(cuda, ove
         assert it == its
         assert abs(r - rs) <= 1e-9 * rs
         assert rel_l2(W.cpu().numpy(), Ws.cpu().numpy()) < 1e-12
+
+
+@pytest.mark.parametrize("precision", [capi.F64, capi.F32])
+def test_batch_replay_length_changes_nothing(cuda, precision):
+    """Residuals finished after every step (a replay longer than the shortest
+    period) and once per replay (at most one period each; lengths that divide
+    the periods and not) give the same bits, update counts and residuals."""
+    torch = cuda
+    probs = _problems()
+    ref = None
+    nts = None
+    for steps in (1, 7, 16, None):
+        b = capi.Batch(probs, precision)
+        nts = [b.info(k)[1] for k in range(b.n)]
+        steps = steps if steps is not None else min(nts) + 3
+        print(f"batch replay of {steps} steps, periods {nts}", flush=True)
+        b.solve(1e-4, 12, steps_per_graph=steps)
+        got = []
+        for k in range(b.n):
+            W = torch.empty(b.info(k)[0], dtype=torch.float64, device="cuda")
+            got.append(b.result(k, W) + (W,))
+        if ref is None:
+            ref = got
+        for (i0, r0, W0), (i1, r1, W1) in zip(ref, got):
+            assert i0 == i1 and r0 == r1 and torch.equal(W0, W1)

@@ -38,10 +38,6 @@
 
 namespace {
 
-struct BatchBlock {
-    int prob, N, e0, nloc, gid;  // gid: index in the full table (residual partials)
-};
-
 struct BatchProb {
     long long soff;  // offset of the problem's state in the concatenated arrays
     long long coff;  // filter-coefficient table offset (nt + 1 entries)
@@ -49,6 +45,13 @@ struct BatchProb {
     const double* basis;
     double ha, hb;
     int eoff, nel, N, nt, blk_off, nblk;
+};
+
+// One workgroup's work, with its problem's record beside it: a launch reads it
+// in one dependent load instead of two before its state loads.
+struct BatchBlock {
+    int prob, N, e0, nloc, gid;  // gid: index in the full table (residual partials)
+    BatchProb pr;
 };
 
 struct BatchArgs {
@@ -75,23 +78,26 @@ struct BatchArgs {
     const long long* G;
     double rk_a, rk_b;
     int stage;
+    int step;        // this launch's step after *G
+    int check;       // 1: problems may retire between the launches of one replay
 };
 
 constexpr int kBT = 256;  // threads per workgroup
 
+// LDS of one workgroup of order n
 template <typename R>
-constexpr size_t max_op_lds()
+size_t op_lds(int n)
 {
-    size_t m = 0;
-    m = std::max(m, wdg::OpLds<2, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<3, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<4, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<5, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<6, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<7, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<8, R, true, true>::bytes);
-    m = std::max(m, wdg::OpLds<9, R, true, true>::bytes);
-    return m;
+    switch (n) {
+    case 2: return wdg::OpLds<2, R, true, true>::bytes;
+    case 3: return wdg::OpLds<3, R, true, true>::bytes;
+    case 4: return wdg::OpLds<4, R, true, true>::bytes;
+    case 5: return wdg::OpLds<5, R, true, true>::bytes;
+    case 6: return wdg::OpLds<6, R, true, true>::bytes;
+    case 7: return wdg::OpLds<7, R, true, true>::bytes;
+    case 8: return wdg::OpLds<8, R, true, true>::bytes;
+    default: return wdg::OpLds<9, R, true, true>::bytes;
+    }
 }
 
 // KIND 0: RK stage 0, 1: stages 1-3, 2: stage 4 (accumulate, finish periods)
@@ -228,7 +234,7 @@ __device__ __forceinline__ void batch_body(const BatchArgs& a, const BatchBlock&
         }
     }
     if (period_end) {  // uniform per workgroup
-        double* red = reinterpret_cast<double*>(lds + max_op_lds<R>());
+        double* red = reinterpret_cast<double*>(lds);  // the operator's tiles are free
         __syncthreads();
         red[threadIdx.x] = part;
         __syncthreads();
@@ -244,12 +250,22 @@ template <typename R, int KIND>
 __global__ __launch_bounds__(kBT) void batch_stage_kernel(const BatchArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
-    const BatchBlock blk = a.blocks[blockIdx.x];
-    if (!a.active[blk.prob]) return;  // uniform per workgroup
-    const BatchProb pr = a.probs[blk.prob];
-    const long long G = *a.G;
-    const int s = (int)(G % pr.nt);
-    const long long it = G / pr.nt;
+    // each XCD walks one contiguous run of workgroups, so that neighbouring
+    // elements of a problem share its L2
+    const BatchBlock blk = a.blocks[wdg::xcd_block(blockIdx.x, gridDim.x)];
+    if (a.check && !a.active[blk.prob]) return;  // uniform per workgroup
+    const BatchProb& pr = blk.pr;
+    const long long G = *a.G + a.step;
+    // G = it nt + s; the 64-bit division only where G needs it
+    int s;
+    long long it;
+    if (G < (1LL << 31)) {
+        it = (unsigned)G / (unsigned)pr.nt;
+        s = (int)((unsigned)G - (unsigned)it * (unsigned)pr.nt);
+    } else {
+        it = G / pr.nt;
+        s = (int)(G - it * pr.nt);
+    }
     switch (blk.N) {
     case 2: batch_body<2, R, KIND>(a, blk, pr, s, it, G, lds); break;
     case 3: batch_body<3, R, KIND>(a, blk, pr, s, it, G, lds); break;
@@ -264,19 +280,20 @@ __global__ __launch_bounds__(kBT) void batch_stage_kernel(const BatchArgs a)
 }
 
 // One workgroup per problem: finish the residual of problems whose period
-// ended at step G, retire converged ones; the last workgroup advances G.
+// ended in the steps G .. G + steps - 1 (at most one period each), retire
+// converged ones; the last workgroup advances G by steps.
 __global__ __launch_bounds__(kBT) void batch_reduce_kernel(const BatchProb* probs, const int* prob_ids,
                                                            const double* partial, int* active, long long* G,
                                                            unsigned int* done, double* pn, double* hist, int* iters,
                                                            int hist_len, double tol, int max_iter, double* best,
-                                                           int* stall, int stall_window)
+                                                           int* stall, int stall_window, int steps)
 {
     __shared__ double red[kBT];
     const int k = prob_ids[blockIdx.x];
     const long long g = *G;
     const BatchProb pr = probs[k];
-    if (active[k] && (g + 1) % pr.nt == 0) {
-        const long long it = g / pr.nt;
+    const long long it = (g + steps) / pr.nt - 1;  // the last period that has ended by then
+    if (active[k] && (it + 1) * pr.nt > g) {
         double sum = 0.0;
         for (int b = threadIdx.x; b < pr.nblk; b += kBT) sum += partial[pr.blk_off + b];
         red[threadIdx.x] = sum;
@@ -313,7 +330,7 @@ __global__ __launch_bounds__(kBT) void batch_reduce_kernel(const BatchProb* prob
         const unsigned int ticket = atomicAdd(done, 1u);
         if (ticket == gridDim.x - 1) {
             *done = 0u;
-            *G = g + 1;
+            *G = g + steps;
             __threadfence();
         }
     }
@@ -489,11 +506,15 @@ struct wdg_batch_s {
 
 namespace {
 
+// Step `step` after *G; with `steps` > 0 the residuals of that many steps are
+// finished after it.
 template <typename R>
-void launch_step(const wdg_batch_s& b, hipStream_t s, double tol, int max_iter)
+void launch_step(const wdg_batch_s& b, hipStream_t s, double tol, int max_iter, int step, int steps, bool check)
 {
     for (int st = 0; st < 5; ++st) {
-        const BatchArgs a = b.args(st);
+        BatchArgs a = b.args(st);
+        a.step = step;
+        a.check = check ? 1 : 0;
         if (st == 0)
             hipLaunchKernelGGL((batch_stage_kernel<R, 0>), dim3(b.n_run_blocks), dim3(kBT), b.lds, s, a);
         else if (st < 4)
@@ -501,9 +522,10 @@ void launch_step(const wdg_batch_s& b, hipStream_t s, double tol, int max_iter)
         else
             hipLaunchKernelGGL((batch_stage_kernel<R, 2>), dim3(b.n_run_blocks), dim3(kBT), b.lds, s, a);
     }
-    hipLaunchKernelGGL(batch_reduce_kernel, dim3(b.n_run_probs), dim3(kBT), 0, s, b.d_probs, b.d_prob_ids, b.d_partial,
-                       b.d_active, b.d_G, b.d_done, b.d_pn, b.d_hist, b.d_iters, b.hist_len, tol, max_iter, b.d_best,
-                       b.d_stall, b.stall_window);
+    if (steps > 0)
+        hipLaunchKernelGGL(batch_reduce_kernel, dim3(b.n_run_probs), dim3(kBT), 0, s, b.d_probs, b.d_prob_ids, b.d_partial,
+                           b.d_active, b.d_G, b.d_done, b.d_pn, b.d_hist, b.d_iters, b.hist_len, tol, max_iter, b.d_best,
+                           b.d_stall, b.stall_window, steps);
 }
 
 // Tables of the problems still running (host flags), uploaded for the next capture.
@@ -535,7 +557,7 @@ void capture(wdg_batch_s& b, int steps, Fn&& step)
     if (!b.cap) bcheck(hipStreamCreateWithFlags(&b.cap, hipStreamNonBlocking), "hipStreamCreate");
     hipGraph_t gph = nullptr;
     bcheck(hipStreamBeginCapture(b.cap, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    for (int k = 0; k < steps; ++k) step(b.cap);
+    for (int k = 0; k < steps; ++k) step(b.cap, k);
     bcheck(hipStreamEndCapture(b.cap, &gph), "hipStreamEndCapture");
     const hipError_t ie = hipGraphInstantiate(&b.graph, gph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(gph);
@@ -622,7 +644,7 @@ int wdg_hip_batch_create(int n_problems, const wdg_batch_problem* problems, int 
             ctab.push_back(dt);
             const int epb = 256 / NN > 0 ? 256 / NN : 1;
             for (int e0 = 0; e0 < nel; e0 += epb)
-                blocks.push_back(BatchBlock{k, n, e0, std::min(epb, nel - e0), (int)blocks.size()});
+                blocks.push_back(BatchBlock{k, n, e0, std::min(epb, nel - e0), (int)blocks.size(), {}});
             pr.nblk = (int)blocks.size() - pr.blk_off;
             for (int e = 0; e < nel; ++e) {
                 const double* c = &m.corners()[8 * (size_t)e];
@@ -662,7 +684,6 @@ int wdg_hip_batch_create(int n_problems, const wdg_batch_problem* problems, int 
         }
         b->ntot = soff;
         b->nblk = (int)blocks.size();
-        b->all_blocks = blocks;
         b->d_prob_ids = dalloc<int>(n_problems);
         // device arrays
         b->d_blocks = dalloc<BatchBlock>(blocks.size());
@@ -672,7 +693,6 @@ int wdg_hip_batch_create(int n_problems, const wdg_batch_problem* problems, int 
         b->d_info = dalloc<int32_t>(info.size());
         b->d_ctab = dalloc<double>(ctab.size());
         b->d_ftab = dalloc<double>(ftab.size());
-        bcheck(hipMemcpy(b->d_blocks, blocks.data(), sizeof(BatchBlock) * blocks.size(), hipMemcpyHostToDevice), "upload");
         bcheck(hipMemcpy(b->d_basis, basis_all.data(), sizeof(double) * basis_all.size(), hipMemcpyHostToDevice), "upload");
         bcheck(hipMemcpy(b->d_geom, geom.data(), sizeof(double) * geom.size(), hipMemcpyHostToDevice), "upload");
         bcheck(hipMemcpy(b->d_nbr, nbr.data(), sizeof(int32_t) * nbr.size(), hipMemcpyHostToDevice), "upload");
@@ -686,6 +706,8 @@ int wdg_hip_batch_create(int n_problems, const wdg_batch_problem* problems, int 
         bcheck(hipMemcpy(b->d_ctab, ctab.data(), sizeof(double) * ctab.size(), hipMemcpyHostToDevice), "upload");
         bcheck(hipMemcpy(b->d_ftab, ftab.data(), sizeof(double) * ftab.size(), hipMemcpyHostToDevice), "upload");
         for (int k = 0; k < n_problems; ++k) b->probs[k].basis = b->d_basis + basis_off[b->probs[k].N];
+        for (BatchBlock& blk : blocks) blk.pr = b->probs[blk.prob];
+        b->all_blocks = blocks;
         b->d_probs = dalloc<BatchProb>(n_problems);
         bcheck(hipMemcpy(b->d_probs, b->probs.data(), sizeof(BatchProb) * n_problems, hipMemcpyHostToDevice), "upload");
         const size_t sb = b->rsz * (size_t)b->ntot;
@@ -708,7 +730,9 @@ int wdg_hip_batch_create(int n_problems, const wdg_batch_problem* problems, int 
         b->d_done = dalloc<unsigned int>(1);
         bcheck(hipMemset(b->d_warm, 0, sizeof(int) * n_problems), "hipMemset");
         bcheck(hipMemset(b->d_winit, 0, sizeof(double) * b->ntot), "hipMemset");
-        b->lds = (precision == WDG_F32 ? max_op_lds<float>() : max_op_lds<double>()) + kBT * sizeof(double);
+        b->lds = kBT * sizeof(double);  // the residual's partial sums
+        for (const BatchProb& pr : b->probs)
+            b->lds = std::max(b->lds, precision == WDG_F32 ? op_lds<float>(pr.N) : op_lds<double>(pr.N));
         // load vectors, one problem at a time with the single-problem kernels
         double* Fd = dalloc<double>(b->ntot);
         double* d_src = nullptr;
@@ -817,11 +841,19 @@ int wdg_hip_batch_solve(wdg_batch b, double tol, int max_iter, int steps_per_gra
                            b->d_G, b->d_done, b->d_iters, b->d_best, b->d_stall);
         bcheck(hipGetLastError(), "batch reset");
         std::vector<int> act(b->nprob, 1), run(b->nprob, 1);
-        auto step = [&](hipStream_t cs) {
+        // Where no period is shorter than a replay, each problem ends at most
+        // one period per replay and its iterate does not change again before
+        // the next one, so the residuals are finished once per replay (a launch
+        // per step took 5.5 of 98 us); otherwise after every step.
+        int min_nt = b->probs[0].nt;
+        for (const BatchProb& pr : b->probs) min_nt = std::min(min_nt, pr.nt);
+        const bool once = min_nt >= steps_per_graph;
+        auto step = [&](hipStream_t cs, int k) {
+            const int at = once ? k : 0, fin = !once ? 1 : (k + 1 == steps_per_graph ? steps_per_graph : 0);
             if (b->prec == WDG_F32)
-                launch_step<float>(*b, cs, tol, max_iter);
+                launch_step<float>(*b, cs, tol, max_iter, at, fin, !once);
             else
-                launch_step<double>(*b, cs, tol, max_iter);
+                launch_step<double>(*b, cs, tol, max_iter, at, fin, !once);
         };
         compact(*b, run, s);
         capture(*b, steps_per_graph, step);
