@@ -217,3 +217,31 @@ def test_exact_advection_wave_matrices_equal_exact_wave_action(cuda, leg):
     gx.action(u, y2)
     torch.cuda.synchronize()
     assert float(torch.linalg.norm(y1 - y2) / torch.linalg.norm(y2)) < TOL
+
+
+@BASES
+@pytest.mark.parametrize("n", [3, 6])
+def test_fused_action_equals_general_path(cuda, n, leg):
+    """Up to three variables run the fused action kernel, more the volume and
+    face kernels: a system of four uncoupled scalars with their own per-node
+    velocities against each scalar alone."""
+    torch = cuda
+    v, e = mesh_case("skewed6x5")
+    mesh = capi.Mesh(v, e)
+    wave = capi.Wave2D(mesh, n, None, basis=capi.GAUSS_LEGENDRE if leg else capi.GAUSS_LOBATTO)
+    npts = n * n * mesh.n_elem
+    rng = np.random.default_rng(n)
+    c = rng.standard_normal((4, npts, 2))
+    A4 = np.zeros((npts, 2, 4, 4))  # (node, direction, column, row): column-major per node
+    for k in range(4):
+        A4[:, :, k, k] = c[k]
+    u = rng.standard_normal((npts, 4))
+    y4 = torch.zeros(4 * npts, dtype=torch.float64, device="cuda")
+    capi.Advection(wave, 4, A4.reshape(-1), False).action(torch.tensor(u.reshape(-1), device="cuda"), y4)
+    y4 = y4.cpu().numpy().reshape(npts, 4)
+    for k in range(4):
+        y = torch.ones(npts, dtype=torch.float64, device="cuda")
+        adv = capi.Advection(wave, 1, np.ascontiguousarray(c[k]).reshape(-1), False)
+        adv.action(torch.tensor(np.ascontiguousarray(u[:, k]), device="cuda"), y)
+        torch.cuda.synchronize()
+        assert rel_l2(y.cpu().numpy() - 1.0, y4[:, k]) < 1e-12

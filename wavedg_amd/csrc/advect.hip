@@ -115,6 +115,169 @@ __global__ __launch_bounds__(64) void advect_face_kernel(const double* __restric
     }
 }
 
+// Advection<true>::action in one pass for up to three variables: the volume
+// term of divf_linear_kernel and the interior edge fluxes of
+// advect_face_kernel, so y is read and written once and u, its traces and
+// the coefficients come in one round of loads.  One thread per node,
+// Shape<N>::EPB whole elements per workgroup; face lanes (4 N per element)
+// leave their contributions in LDS and every node adds the sides that reach
+// it, sides 0 and 2 before 1 and 3.  Boundary sides add nothing here.
+// LEG: Gauss-Legendre basis (P = phi_m(-1)).  Bound by memory (y twice, u,
+// the coefficient, H and, for LEG, the neighbours' lines through L2) and, at
+// small sizes, by the launch that it saves.  Scalar, per-node coefficient,
+// volume + face kernels and now: 320 x 240 P = 5 Gauss-Legendre 61 -> 31 us,
+// 256^2 P = 7 Gauss-Lobatto 65 -> 34 us, 64^2 P = 3 11 -> 9 us.
+template <int N, int NV, bool LEG>
+__global__ __launch_bounds__(Shape<N>::NT) void advect_action_kernel(const DivFArgs a, const int32_t* __restrict__ nbr,
+                                                                     const int32_t* __restrict__ info,
+                                                                     const double* __restrict__ H)
+{
+    constexpr int NN = N * N, EPB = Shape<N>::EPB, NF = 4 * N, V2 = NV * NV;
+    constexpr int FP = (NF + NN - 1) / NN;  // face points per thread
+    static_assert(EPB * NN >= 3 * N, "one round of threads loads the tables");
+    __shared__ double s_u[EPB * NV * NN], s_F[EPB * NV * NN], s_G[EPB * NV * NN];
+    __shared__ double s_f[EPB * (NF + 1) * NV];  // slot NF of an element: zeros
+    __shared__ double s_D[NN], s_x[3 * N];       // x, w, P
+    const double* __restrict__ u = static_cast<const double*>(a.u);
+    const int tid = threadIdx.x, el = tid / NN, node = tid - el * NN, i = node % N, j = node / N;
+    const int e0 = xcd_block(blockIdx.x, gridDim.x) * EPB, nloc = min(EPB, a.nel - e0);
+    const bool active = el < nloc;
+    const int e = e0 + (active ? el : 0);
+    // every load of the pass before the first wait
+    const size_t at = (size_t)NV * (node + (size_t)NN * e);
+    double uv[NV], yv[NV], An[2 * V2];
+    double* const y = static_cast<double*>(a.out) + at;
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+        uv[c] = u[at + c];
+        yv[c] = y[c];
+    }
+    if (a.Anode) {
+#pragma unroll
+        for (int q = 0; q < 2 * V2; ++q) An[q] = a.Anode[2 * NV * at + q];
+    } else {
+#pragma unroll
+        for (int c = 0; c < NV; ++c)
+#pragma unroll
+            for (int d = 0; d < NV; ++d) {
+                An[d + NV * c] = a.A[d + kMaxVar * c];
+                An[V2 + d + NV * c] = a.B[d + kMaxVar * c];
+            }
+    }
+    const double* gq = a.geom + 6 * (size_t)e;  // ax, ay, cx, cy, hx, hy of the bilinear map
+    const double g0 = gq[0], g1 = gq[1], g2 = gq[2], g3 = gq[3], g4 = gq[4], g5 = gq[5];
+    double ub[FP][NV], Hk[FP][2 * V2];
+    bool on[FP];
+#pragma unroll
+    for (int p = 0; p < FP; ++p) {
+        const int f = node + p * NN, s = f / N, k = f - s * N;
+        on[p] = false;
+#pragma unroll
+        for (int c = 0; c < NV; ++c) ub[p][c] = 0.0;
+        if (!active || f >= NF) continue;
+        const int nb = nbr[4 * (size_t)e + s], inf = info[4 * (size_t)e + s];
+        if (nb < 0) continue;
+        on[p] = true;
+        const double* h = H + (((size_t)e * 4 + s) * N + k) * 2 * V2;
+#pragma unroll
+        for (int q = 0; q < 2 * V2; ++q) Hk[p][q] = h[q];
+        const int ns = inf & 3, kk = ((inf >> 2) & 1) ? (N - 1 - k) : k;
+        const double* q = u + (size_t)NV * ((size_t)nb * NN + side_node<N>(ns, kk));
+        if constexpr (LEG) {
+            const int st = NV * inward_stride<N>(ns);
+            const double* P = a.basis + 2 * N + NN;
+#pragma unroll
+            for (int m = 0; m < N; ++m)
+#pragma unroll
+                for (int c = 0; c < NV; ++c) ub[p][c] = fma(P[m], q[c + m * st], ub[p][c]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < NV; ++c) ub[p][c] = q[c];
+        }
+    }
+    if (tid < NN) s_D[tid] = a.basis[2 * N + tid];
+    if (tid < 2 * N) s_x[tid] = a.basis[tid];
+    if (LEG && tid < N) s_x[2 * N + tid] = a.basis[2 * N + NN + tid];
+    double* const U = s_u + el * NV * NN;
+#pragma unroll
+    for (int c = 0; c < NV; ++c) U[NV * node + c] = uv[c];
+    __syncthreads();
+    {
+        const double xi = s_x[i], eta = s_x[j], wij = s_x[N + i] * s_x[N + j];
+        const double Yx = (g1 + g5 * eta) * wij, Xx = (g0 + g4 * eta) * wij;
+        const double Ye = (g3 + g5 * xi) * wij, Xe = (g2 + g4 * xi) * wij;
+#pragma unroll
+        for (int d = 0; d < NV; ++d) {
+            double fx = 0.0, fy = 0.0;
+#pragma unroll
+            for (int c = 0; c < NV; ++c) {
+                fx = fma(An[d + NV * c], uv[c], fx);
+                fy = fma(An[V2 + d + NV * c], uv[c], fy);
+            }
+            s_F[(el * NV + d) * NN + j * N + i] = Ye * fx - Xe * fy;
+            s_G[(el * NV + d) * NN + i * N + j] = Xx * fy - Yx * fx;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < FP; ++p) {
+        const int f = node + p * NN, s = f / N, k = f - s * N;
+        if (f >= NF) continue;
+        double acc[NV];
+#pragma unroll
+        for (int d = 0; d < NV; ++d) acc[d] = 0.0;
+        if (on[p]) {
+            double ua[NV];
+            const double* q = U + NV * side_node<N>(s, k);
+            if constexpr (LEG) {
+                const int st = NV * inward_stride<N>(s);
+#pragma unroll
+                for (int c = 0; c < NV; ++c) ua[c] = 0.0;
+#pragma unroll
+                for (int m = 0; m < N; ++m)
+#pragma unroll
+                    for (int c = 0; c < NV; ++c) ua[c] = fma(s_x[2 * N + m], q[c + m * st], ua[c]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < NV; ++c) ua[c] = q[c];
+            }
+#pragma unroll
+            for (int d = 0; d < NV; ++d)
+#pragma unroll
+                for (int c = 0; c < NV; ++c) {
+                    acc[d] = fma(Hk[p][d + NV * c], ua[c], acc[d]);
+                    acc[d] = fma(Hk[p][V2 + d + NV * c], ub[p][c], acc[d]);
+                }
+        }
+#pragma unroll
+        for (int d = 0; d < NV; ++d) s_f[(el * (NF + 1) + f) * NV + d] = acc[d];
+    }
+    if (node < NV) s_f[(el * (NF + 1) + NF) * NV + node] = 0.0;
+    __syncthreads();
+    if (!active) return;
+    const double* S = s_f + el * (NF + 1) * NV;
+#pragma unroll
+    for (int d = 0; d < NV; ++d) {
+        const double* Fr = s_F + (el * NV + d) * NN + j * N;
+        const double* Gc = s_G + (el * NV + d) * NN + i * N;
+        double r = 0.0;
+#pragma unroll
+        for (int l = 0; l < N; ++l) {
+            r = fma(s_D[l + N * i], Fr[l], r);
+            r = fma(s_D[l + N * j], Gc[l], r);
+        }
+        if constexpr (LEG) {
+            const double* P = s_x + 2 * N;
+            r += P[j] * S[i * NV + d] + P[N - 1 - i] * S[(N + j) * NV + d] + P[N - 1 - j] * S[(2 * N + i) * NV + d] +
+                 P[i] * S[(3 * N + j) * NV + d];
+        } else {
+            const int fa = j == 0 ? i : (j == N - 1 ? 2 * N + i : NF);
+            const int fb = i == N - 1 ? N + j : (i == 0 ? 3 * N + j : NF);
+            r += S[fa * NV + d] + S[fb * NV + d];
+        }
+        y[d] = yv[d] + r;
+    }
+}
+
 // Compressible Euler flux and local Lax-Friedrichs flux of examples/cl2d.cpp
 // (F :57-81, speed :84-96, numerical_flux :98-111).
 __device__ __forceinline__ void euler_fg(double gamma, const double* q, double* f, double* g, double& speed)
@@ -528,6 +691,44 @@ void launch_euler_face(int n, double gamma, const double* q, double* y, const do
     default: break;
     }
 #undef WDG_EULER_CASE
+}
+
+bool launch_advect_action(int n, const DivFArgs& a, const int32_t* nbr, const int32_t* info, const double* H, bool leg,
+                          hipStream_t s)
+{
+    if (a.nv < 1 || a.nv > 3) return false;
+    if (a.nel <= 0) return true;
+#define WDG_ACT_NV(NV_, VAR_)                                                                                      \
+    if (leg)                                                                                                       \
+        hipLaunchKernelGGL((advect_action_kernel<NV_, VAR_, true>), grid, block, 0, s, a, nbr, info, H);           \
+    else                                                                                                           \
+        hipLaunchKernelGGL((advect_action_kernel<NV_, VAR_, false>), grid, block, 0, s, a, nbr, info, H);
+#define WDG_ACT_CASE(NV_)                                                                                          \
+    case NV_: {                                                                                                    \
+        const dim3 grid((a.nel + Shape<NV_>::EPB - 1) / Shape<NV_>::EPB), block(Shape<NV_>::NT);                   \
+        if (a.nv == 1) {                                                                                           \
+            WDG_ACT_NV(NV_, 1)                                                                                     \
+        } else if (a.nv == 2) {                                                                                    \
+            WDG_ACT_NV(NV_, 2)                                                                                     \
+        } else {                                                                                                   \
+            WDG_ACT_NV(NV_, 3)                                                                                     \
+        }                                                                                                          \
+        break;                                                                                                     \
+    }
+    switch (n) {
+        WDG_ACT_CASE(2)
+        WDG_ACT_CASE(3)
+        WDG_ACT_CASE(4)
+        WDG_ACT_CASE(5)
+        WDG_ACT_CASE(6)
+        WDG_ACT_CASE(7)
+        WDG_ACT_CASE(8)
+        WDG_ACT_CASE(9)
+    default: return false;
+    }
+#undef WDG_ACT_CASE
+#undef WDG_ACT_NV
+    return true;
 }
 
 void launch_advect_face(int n, int nv, const double* u, double* y, const int32_t* nbr, const int32_t* info,

@@ -2064,6 +2064,11 @@ static int advection_launch(wdg_advection adv, const void* d_u, void* d_divF, bo
             std::memcpy(a.A, adv->A0, sizeof(a.A));
             std::memcpy(a.B, adv->A1, sizeof(a.B));
             a.Anode = adv->d_Anode;
+            if (interior && !boundary &&
+                wdg::launch_advect_action(op->n, a, op->d_nbr, op->d_info, adv->d_H, op->leg != 0, s)) {
+                hip_check(hipGetLastError(), "advection kernel launch");
+                return;
+            }
             wdg::launch_divf_linear(op->n, 0, a, s);
         }
         wdg::launch_advect_face(op->n, adv->nv, static_cast<const double*>(d_u), static_cast<double*>(d_divF),

@@ -856,6 +856,11 @@ void launch_divf_linear(int n, int f32, const DivFArgs& a, hipStream_t s);
 // P: face interpolation phi_m(-1) of a Gauss-Legendre basis, or null.
 void launch_advect_face(int n, int nv, const double* u, double* y, const int32_t* nbr, const int32_t* info,
                         const double* H, const double* P, int nel, int interior, int boundary, hipStream_t s);
+// Both terms of Advection<true>::action in one kernel, for up to three
+// variables (false: not covered; two kernels do it).  a as for
+// launch_divf_linear, H as for launch_advect_face.
+bool launch_advect_action(int n, const DivFArgs& a, const int32_t* nbr, const int32_t* info, const double* H, bool leg,
+                          hipStream_t s);
 // Advection<false> (advect.hip): volume term on nq_volume^2 points with the
 // metric-weighted coefficient table op (2, nv, nv, nq, nq, nel) and tabv = P,
 // D (nq, n); face terms on nq_edge points with Hq (2, nv, nv) per (element,
