@@ -32,7 +32,8 @@ __global__ __launch_bounds__(64) void advect_face_kernel(const double* __restric
                                                          const int32_t* __restrict__ nbr,
                                                          const int32_t* __restrict__ info,
                                                          const double* __restrict__ H, const double* __restrict__ P,
-                                                         int nv, int nel, int interior, int boundary)
+                                                         int nv, int nel, const int32_t* __restrict__ list,
+                                                         int interior, int boundary)
 {
     constexpr int NN = N * N, NF = 4 * N;
     constexpr int kF = NF * kMaxVar > 64 ? NF * kMaxVar : 64;
@@ -41,22 +42,24 @@ __global__ __launch_bounds__(64) void advect_face_kernel(const double* __restric
     const int per = NF * nv, E = per < 64 ? 64 / per : 1;
     const int tid = threadIdx.x, e0 = blockIdx.x * E, vn = nv * NN, v2 = nv * nv;
     const int nloc = nel - e0 < E ? nel - e0 : E;
+    auto elem = [&](int el) { return list ? list[e0 + el] : e0 + el; };
     if (tid < E) s_any[tid] = 0;
-    {
-        // a workgroup whose elements have no side in this launch (e.g. away
-        // from the boundary) has nothing to do
+    if (!list) {
+        // a workgroup whose elements have no side in this launch has nothing to do
         bool act = false;
         for (int t = tid; t < 4 * nloc; t += 64) {
             const int nb = nbr[4 * ((size_t)e0 + t / 4) + (t % 4)];
             act = act || (nb >= 0 ? interior != 0 : boundary != 0);
         }
         if (!__syncthreads_or(act)) return;
+    } else {
+        __syncthreads();  // s_any is clear before a lane sets it
     }
     for (int it = tid; it < E * per; it += 64) {
         const int el = it / per, r = it - el * per, f = r / nv, d = r - f * nv, s = f / N, k = f - s * N;
-        const int e = e0 + el;
         double acc = 0.0;
         if (el < nloc) {
+            const int e = elem(el);
             const int nb = nbr[4 * (size_t)e + s], inf = info[4 * (size_t)e + s];
             const bool is_int = nb >= 0;
             if (is_int ? interior : boundary) {
@@ -93,10 +96,10 @@ __global__ __launch_bounds__(64) void advect_face_kernel(const double* __restric
         s_f[(el * NF + f) * nv + d] = acc;
     }
     __syncthreads();
-    double* yb = y + (size_t)e0 * vn;
     for (int t = tid; t < nloc * vn; t += 64) {
         const int el = t / vn, r = t - el * vn, node = r / nv, d = r - node * nv;
         if (!s_any[el]) continue;
+        double* yb = y + (size_t)elem(el) * vn;
         const int i = node % N, j = node / N;
         const double* F = s_f + el * NF * nv + d;
         double add;
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(64) void advect_face_kernel(const double* __restric
             if (j == N - 1) add += F[(2 * N + i) * nv];
             if (i == 0) add += F[(3 * N + j) * nv];
         }
-        yb[t] += add;
+        yb[r] += add;
     }
 }
 
@@ -322,36 +325,62 @@ __device__ __forceinline__ void trace4(const double* p, int s, const double* P, 
 // (element, side, side node), all four sides at once, E = 64 / 4N elements
 // per workgroup; each lane leaves its contribution in LDS and the nodes then
 // add their sides in side order 0..3 (corner nodes two), so every output has
-// one writer.  A Gauss-Legendre basis (P non-null) interpolates the traces
-// along the element and lifts every side back along its lines with P.
-template <int N>
+// one writer.  A Gauss-Legendre basis (LEG) interpolates the traces along the
+// element and lifts every side back along its lines with P.  Bound by memory:
+// on a Gauss-Lobatto basis the lanes walk the boundary nodes alone and load
+// their y before the fluxes (401 x 399 P = 4: 91 -> 80 us against walking all
+// nodes after them).  A boundary launch visits a list of the boundary elements.
+template <int N, bool LEG>
 __global__ __launch_bounds__(64) void euler_face_kernel(double gamma, const double* __restrict__ q,
                                                         double* __restrict__ y, const double* __restrict__ geom,
                                                         const int32_t* __restrict__ nbr,
                                                         const int32_t* __restrict__ info,
                                                         const double* __restrict__ basis,
-                                                        const double* __restrict__ P, int nel, int interior,
-                                                        int boundary)
+                                                        const double* __restrict__ P, int nel,
+                                                        const int32_t* __restrict__ list, int interior, int boundary)
 {
     constexpr int NN = N * N, NF = 4 * N, E = 64 / NF > 0 ? 64 / NF : 1;
+    constexpr int NB = 4 * (N - 1) * 4;               // values of an element's boundary nodes
+    constexpr int NI = LEG ? 1 : (E * NB + 63) / 64;  // of them per lane
     __shared__ double s_f[E * NF * 4];  // each side node's contribution, this element's order
     __shared__ int s_any[E];            // the element has a side in this launch
     const int tid = threadIdx.x, e0 = blockIdx.x * E;
     const int nloc = nel - e0 < E ? nel - e0 : E;
+    auto elem = [&](int el) { return list ? list[e0 + el] : e0 + el; };
     if (tid < E) s_any[tid] = 0;
-    {
-        // a workgroup whose elements have no side in this launch (e.g. away
-        // from the boundary) has nothing to do
+    if (!list) {
+        // a workgroup whose elements have no side in this launch has nothing to do
         bool act = false;
         for (int t = tid; t < 4 * nloc; t += 64) {
             const int nb = nbr[4 * ((size_t)e0 + t / 4) + (t % 4)];
             act = act || (nb >= 0 ? interior != 0 : boundary != 0);
         }
         if (!__syncthreads_or(act)) return;
+    } else {
+        __syncthreads();  // s_any is clear before a lane sets it
     }
-    const int el = tid / NF, f = tid - el * NF, s = f / N, k = f - (f / N) * N, e = e0 + el;
+    // Gauss-Lobatto: the sides reach the boundary nodes alone.  This lane's
+    // values of y, loaded before the fluxes: node b of an element's boundary,
+    // counter-clockwise from corner 0, is node r = b % (N - 1) of side
+    // b / (N - 1), and its corners (r = 0) also end the side before.
+    double yv[NI];
+    size_t yat[NI];
+    if constexpr (!LEG) {
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            const int t = tid + 64 * q, el = t / NB, w = t - el * NB, d = w & 3, b = w >> 2;
+            const int s = b / (N - 1), r = b - s * (N - 1);
+            const int i = s == 0 ? r : s == 1 ? N - 1 : s == 2 ? N - 1 - r : 0;
+            const int j = s == 0 ? 0 : s == 1 ? r : s == 2 ? N - 1 : N - 1 - r;
+            if (el >= nloc) continue;
+            yat[q] = (size_t)elem(el) * 4 * NN + 4 * (i + N * j) + d;
+            yv[q] = y[yat[q]];
+        }
+    }
+    const int el = tid / NF, f = tid - el * NF, s = f / N, k = f - (f / N) * N;
     double c[4] = {0.0, 0.0, 0.0, 0.0};
     if (tid < E * NF && el < nloc) {
+        const int e = elem(el);
         const int nb = nbr[4 * (size_t)e + s], inf = info[4 * (size_t)e + s];
         const bool is_int = nb >= 0;
         if (is_int ? interior : boundary) {
@@ -388,24 +417,30 @@ __global__ __launch_bounds__(64) void euler_face_kernel(double gamma, const doub
         for (int d = 0; d < 4; ++d) s_f[(el * NF + f) * 4 + d] = c[d];
     }
     __syncthreads();
-    for (int t = tid; t < nloc * 4 * NN; t += 64) {
-        const int el2 = t / (4 * NN), r = t - el2 * 4 * NN, node = r / 4, d = r - node * 4;
-        if (!s_any[el2]) continue;
-        const int i = node % N, j = node / N;
-        const double* F = s_f + el2 * NF * 4 + d;
-        double add;
-        if (P) {
-            add = P[j] * F[(0 * N + i) * 4] + P[N - 1 - i] * F[(1 * N + j) * 4] + P[N - 1 - j] * F[(2 * N + i) * 4] +
-                  P[i] * F[(3 * N + j) * 4];
-        } else {
-            if (!(i == 0 || j == 0 || i == N - 1 || j == N - 1)) continue;  // no side reaches an inner node
-            add = 0.0;
-            if (j == 0) add += F[(0 * N + i) * 4];
-            if (i == N - 1) add += F[(1 * N + j) * 4];
-            if (j == N - 1) add += F[(2 * N + i) * 4];
-            if (i == 0) add += F[(3 * N + j) * 4];
+    if constexpr (LEG) {
+        for (int t = tid; t < nloc * 4 * NN; t += 64) {
+            const int el2 = t / (4 * NN), r = t - el2 * 4 * NN, node = r / 4, d = r - node * 4;
+            if (!s_any[el2]) continue;
+            const int i = node % N, j = node / N;
+            const double* F = s_f + el2 * NF * 4 + d;
+            y[(size_t)elem(el2) * 4 * NN + r] += P[j] * F[(0 * N + i) * 4] + P[N - 1 - i] * F[(1 * N + j) * 4] +
+                                                 P[N - 1 - j] * F[(2 * N + i) * 4] + P[i] * F[(3 * N + j) * 4];
         }
-        y[(size_t)(e0 + el2) * 4 * NN + r] += add;
+    } else {
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            const int t = tid + 64 * q, el2 = t / NB, w = t - el2 * NB, d = w & 3, b = w >> 2;
+            const int s2 = b / (N - 1), r = b - s2 * (N - 1);
+            if (el2 >= nloc || !s_any[el2]) continue;
+            const double* F = s_f + el2 * NF * 4 + d;
+            // sides 2 and 3 are numbered along i and j, against the walk
+            double add = F[(s2 * N + (s2 < 2 ? r : N - 1 - r)) * 4];
+            if (r == 0) {
+                const int sp = (s2 + 3) & 3;
+                add += F[(sp * N + (sp < 2 ? N - 1 : 0)) * 4];
+            }
+            y[yat[q]] = yv[q] + add;
+        }
     }
 }
 
@@ -669,16 +704,22 @@ void launch_linear_functional(int n, int nq, int nv, const double* corners, cons
 static int euler_elems(int n) { return 64 / (4 * n) > 0 ? 64 / (4 * n) : 1; }
 
 void launch_euler_face(int n, double gamma, const double* q, double* y, const double* geom, const int32_t* nbr,
-                       const int32_t* info, const double* basis, const double* P, int nel, int interior, int boundary,
-                       hipStream_t s)
+                       const int32_t* info, const double* basis, const double* P, int nel, const int32_t* list,
+                       int interior, int boundary, hipStream_t s)
 {
     if (nel <= 0) return;
     const dim3 block(64);
 #define WDG_EULER_CASE(NV_)                                                                                   \
-    case NV_:                                                                                                 \
-        hipLaunchKernelGGL(euler_face_kernel<NV_>, dim3((nel + euler_elems(NV_) - 1) / euler_elems(NV_)), block, 0, \
-                           s, gamma, q, y, geom, nbr, info, basis, P, nel, interior, boundary);               \
-        break;
+    case NV_: {                                                                                               \
+        const dim3 grid((nel + euler_elems(NV_) - 1) / euler_elems(NV_));                                     \
+        if (P)                                                                                                \
+            hipLaunchKernelGGL((euler_face_kernel<NV_, true>), grid, block, 0, s, gamma, q, y, geom, nbr,     \
+                               info, basis, P, nel, list, interior, boundary);                                \
+        else                                                                                                  \
+            hipLaunchKernelGGL((euler_face_kernel<NV_, false>), grid, block, 0, s, gamma, q, y, geom, nbr,    \
+                               info, basis, P, nel, list, interior, boundary);                                \
+        break;                                                                                                \
+    }
     switch (n) {
         WDG_EULER_CASE(2)
         WDG_EULER_CASE(3)
@@ -732,15 +773,16 @@ bool launch_advect_action(int n, const DivFArgs& a, const int32_t* nbr, const in
 }
 
 void launch_advect_face(int n, int nv, const double* u, double* y, const int32_t* nbr, const int32_t* info,
-                        const double* H, const double* P, int nel, int interior, int boundary, hipStream_t s)
+                        const double* H, const double* P, int nel, const int32_t* list, int interior, int boundary,
+                        hipStream_t s)
 {
     if (nel <= 0 || nv < 1 || nv > kMaxVar) return;
     const int per = 4 * n * nv, E = per < 64 ? 64 / per : 1;  // advect_face_kernel's elements per workgroup
     const dim3 grid((nel + E - 1) / E), block(64);
 #define WDG_ADVECT_CASE(NV_)                                                                                  \
     case NV_:                                                                                                 \
-        hipLaunchKernelGGL(advect_face_kernel<NV_>, grid, block, 0, s, u, y, nbr, info, H, P, nv, nel, interior, \
-                           boundary);                                                                         \
+        hipLaunchKernelGGL(advect_face_kernel<NV_>, grid, block, 0, s, u, y, nbr, info, H, P, nv, nel, list,    \
+                           interior, boundary);                                                               \
         break;
     switch (n) {
         WDG_ADVECT_CASE(2)

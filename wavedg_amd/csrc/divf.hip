@@ -124,7 +124,100 @@ void launch_n(int f32, const DivFArgs& a, hipStream_t s)
 #undef WDG_DIVF_VS
 }
 
+// M = w_i w_j det J per node (MassMatrix<true>, MassMatrix.cpp:6-82).  One
+// thread per node with its NV values contiguous (NV = 0: any number, in a
+// loop), Shape<N>::EPB whole elements per workgroup.  Bound by memory, x read
+// and y written once; a thread per node of a run-time order spent its time in
+// 64-bit index divisions (401 x 399 P = 4, four variables 80 -> 58 us; 320 x 240
+// P = 5, one variable 17 -> 13 us with paired corner loads and the basis in LDS).
+template <int N, typename R, int NV>
+__global__ __launch_bounds__(Shape<N>::NT) void mass_kernel(const R* x, R* y, const double* __restrict__ corners,
+                                                            const double* __restrict__ basis, int nel, int nvar,
+                                                            int inv)
+{
+    constexpr int NN = N * N, EPB = Shape<N>::EPB;
+    __shared__ double s_xw[2 * N];
+    const int nv = NV ? NV : nvar;
+    const int tid = threadIdx.x, el = tid / NN, node = tid - el * NN, i = node % N, j = node / N;
+    const int e = blockIdx.x * EPB + el;
+    const bool active = e < nel;
+    const int ec = active ? e : nel - 1;
+    const size_t at = (size_t)nv * (node + (size_t)NN * ec);
+    R v[NV ? NV : 1];
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int d = 0; d < NV; ++d) v[d] = x[at + d];
+    }
+    // few, wide loads: their issue is what bounds one value per node
+    const double2* cp = reinterpret_cast<const double2*>(corners) + 4 * (size_t)ec;
+    const double2 p0 = cp[0], p1 = cp[1], p2 = cp[2], p3 = cp[3];
+    const double c[8] = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
+    if (tid < 2 * N) s_xw[tid] = basis[tid];
+    __syncthreads();
+    if (!active) return;
+    const double xi = s_xw[i], eta = s_xw[j];
+    const double J0 = 0.25 * ((1.0 - eta) * (c[2] - c[0]) + (1.0 + eta) * (c[4] - c[6]));
+    const double J1 = 0.25 * ((1.0 - eta) * (c[3] - c[1]) + (1.0 + eta) * (c[5] - c[7]));
+    const double J2 = 0.25 * ((1.0 - xi) * (c[6] - c[0]) + (1.0 + xi) * (c[4] - c[2]));
+    const double J3 = 0.25 * ((1.0 - xi) * (c[7] - c[1]) + (1.0 + xi) * (c[5] - c[3]));
+    const double m = s_xw[N + i] * s_xw[N + j] * (J0 * J3 - J1 * J2);
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int d = 0; d < NV; ++d) y[at + d] = inv ? (R)((double)v[d] / m) : (R)(m * (double)v[d]);
+    } else {
+        for (int d = 0; d < nv; ++d) {  // x and y may alias (in-place inverse)
+            const double t = (double)x[at + d];
+            y[at + d] = inv ? (R)(t / m) : (R)(m * t);
+        }
+    }
+}
+
+template <int N, typename R>
+void launch_mass_n(const void* x, void* y, const double* corners, const double* basis, int nel, int nv, int inv,
+                   hipStream_t s)
+{
+    const dim3 grid((nel + Shape<N>::EPB - 1) / Shape<N>::EPB), block(Shape<N>::NT);
+#define WDG_MASS_NV(NV_)                                                                                   \
+    hipLaunchKernelGGL((mass_kernel<N, R, NV_>), grid, block, 0, s, static_cast<const R*>(x),              \
+                       static_cast<R*>(y), corners, basis, nel, nv, inv);
+    if (nv == 1) {
+        WDG_MASS_NV(1)
+    } else if (nv == 3) {
+        WDG_MASS_NV(3)
+    } else if (nv == 4) {
+        WDG_MASS_NV(4)
+    } else {
+        WDG_MASS_NV(0)
+    }
+#undef WDG_MASS_NV
+}
+
 }  // namespace
+
+void launch_mass(int n, int f32, const void* x, void* y, const double* corners, const double* basis, int nel, int nv,
+                 int inv, hipStream_t s)
+{
+    if (nel <= 0) return;
+#define WDG_MASS_CASE(NV_)                                                        \
+    case NV_:                                                                     \
+        if (f32)                                                                  \
+            launch_mass_n<NV_, float>(x, y, corners, basis, nel, nv, inv, s);     \
+        else                                                                      \
+            launch_mass_n<NV_, double>(x, y, corners, basis, nel, nv, inv, s);    \
+        break;
+    switch (n) {
+        WDG_MASS_CASE(2)
+        WDG_MASS_CASE(3)
+        WDG_MASS_CASE(4)
+        WDG_MASS_CASE(5)
+        WDG_MASS_CASE(6)
+        WDG_MASS_CASE(7)
+        WDG_MASS_CASE(8)
+        WDG_MASS_CASE(9)
+    default: break;
+    }
+#undef WDG_MASS_CASE
+}
 
 void launch_divf_linear(int n, int f32, const DivFArgs& a, hipStream_t s)
 {

@@ -134,6 +134,8 @@ struct wdg_wave2d_s {
     float* d_basis32 = nullptr;
     int32_t* d_nbr = nullptr;
     int32_t* d_info = nullptr;
+    int32_t* d_bel = nullptr;  // the elements with a boundary side
+    int n_bel = 0;
     std::map<int, double*> d_lftab;  // LinearFunctional tables per rule size (wdg_hip_linear_functional)
     void* d_fgeo = nullptr;      // FaceGeom<R> per element side (handle precision)
     wdg::FaceNb* d_fnb = nullptr;       // neighbour trace base and flags per element side
@@ -183,6 +185,7 @@ struct wdg_wave2d_s {
         dfree(d_basis32);
         dfree(d_nbr);
         dfree(d_info);
+        dfree(d_bel);
         dfree(d_fgeo);
         dfree(d_fnb);
         for (auto& kv : d_lftab) dfree(kv.second);
@@ -317,31 +320,6 @@ void apply_op(wdg_wave2d op, int kid, const KArgs& a, hipStream_t s)
 }
 
 // ------------------------------------------------------------ small kernels
-template <typename R>
-__global__ void k_mass(const R* x, R* y, const double* __restrict__ corners, const double* __restrict__ basis, int N,
-                       long long nnodes, int nv, int inv)
-{
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nnodes) return;
-    const int NN = N * N;
-    const long long e = q / NN;
-    const int node = (int)(q - e * NN);
-    const int i = node % N, j = node / N;
-    const double* c = corners + 8 * e;
-    const double xi = basis[i], eta = basis[j];
-    const double J0 = 0.25 * ((1.0 - eta) * (c[2] - c[0]) + (1.0 + eta) * (c[4] - c[6]));
-    const double J1 = 0.25 * ((1.0 - eta) * (c[3] - c[1]) + (1.0 + eta) * (c[5] - c[7]));
-    const double J2 = 0.25 * ((1.0 - xi) * (c[6] - c[0]) + (1.0 + xi) * (c[4] - c[2]));
-    const double J3 = 0.25 * ((1.0 - xi) * (c[7] - c[1]) + (1.0 + xi) * (c[5] - c[3]));
-    const double m = basis[N + i] * basis[N + j] * (J0 * J3 - J1 * J2);
-    for (int d = 0; d < nv; ++d) {  // x and y may alias (in-place inverse)
-        if (inv)
-            y[nv * q + d] = (R)((double)x[nv * q + d] / m);
-        else
-            y[nv * q + d] = (R)(m * (double)x[nv * q + d]);
-    }
-}
-
 __device__ double block_sum(double v)
 {
     __shared__ double sh[kRedThreads];
@@ -903,6 +881,17 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
                   "upload nbr");
         hip_check(hipMemcpy(op->d_info, ft.info.data(), sizeof(int32_t) * ft.info.size(), hipMemcpyHostToDevice),
                   "upload info");
+        {
+            std::vector<int32_t> bel;
+            for (int e = 0; e < op->nel; ++e)
+                if (ft.nbr[4 * (size_t)e] < 0 || ft.nbr[4 * (size_t)e + 1] < 0 || ft.nbr[4 * (size_t)e + 2] < 0 ||
+                    ft.nbr[4 * (size_t)e + 3] < 0)
+                    bel.push_back(e);
+            op->n_bel = (int)bel.size();
+            op->d_bel = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * std::max<size_t>(bel.size(), 1)));
+            hip_check(hipMemcpy(op->d_bel, bel.data(), sizeof(int32_t) * bel.size(), hipMemcpyHostToDevice),
+                      "upload boundary elements");
+        }
         hip_check(hipMemcpy(op->d_basis, basis.data(), sizeof(double) * basis.size(), hipMemcpyHostToDevice),
                   "upload basis");
         hip_check(hipMemcpy(op->d_lvtab, lv.data(), sizeof(double) * lv.size(), hipMemcpyHostToDevice),
@@ -1122,7 +1111,6 @@ static int mass_launch(wdg_wave2d op, const void* x, void* y, int inv, void* str
         check_op(op);
         if (!x || !y) fail(WDG_ERR_INVALID, "null device pointer");
         if (nv < 1 || nv > 64) fail(WDG_ERR_INVALID, "n_var out of range 1..64");
-        const long long nn = op->ndof / 3;
         const hipStream_t s = as_stream(stream);
         if (op->exact) {
             if (nv > wdg::DivFArgs::kMaxVar) fail(WDG_ERR_INVALID, "the exact mass matrix takes n_var <= 8");
@@ -1133,12 +1121,7 @@ static int mass_launch(wdg_wave2d op, const void* x, void* y, int inv, void* str
             hip_check(hipGetLastError(), "mass kernel launch");
             return;
         }
-        if (op->prec == WDG_F32)
-            hipLaunchKernelGGL(k_mass<float>, dim3(grid_for(nn)), dim3(256), 0, s, static_cast<const float*>(x),
-                               static_cast<float*>(y), op->d_corners, op->d_basis, op->n, nn, nv, inv);
-        else
-            hipLaunchKernelGGL(k_mass<double>, dim3(grid_for(nn)), dim3(256), 0, s, static_cast<const double*>(x),
-                               static_cast<double*>(y), op->d_corners, op->d_basis, op->n, nn, nv, inv);
+        wdg::launch_mass(op->n, op->prec == WDG_F32, x, y, op->d_corners, op->d_basis, op->nel, nv, inv, s);
         hip_check(hipGetLastError(), "mass kernel launch");
     });
 }
@@ -1765,9 +1748,10 @@ int wdg_hip_edgefluxf2d_euler(wdg_wave2d op, double gamma, int face_type, const 
         if (!d_q || !d_divF) fail(WDG_ERR_INVALID, "null device pointer");
         if (!(gamma > 1.0)) fail(WDG_ERR_INVALID, "gamma must exceed 1");
         if (face_type != WDG_INTERIOR && face_type != WDG_BOUNDARY) fail(WDG_ERR_INVALID, "bad face type");
+        const bool bnd = face_type == WDG_BOUNDARY;  // the boundary elements alone
         wdg::launch_euler_face(op->n, gamma, static_cast<const double*>(d_q), static_cast<double*>(d_divF),
-                               op->d_geom, op->d_nbr, op->d_info, op->d_basis, op->face_interp(), op->nel,
-                               face_type == WDG_INTERIOR ? 1 : 0, face_type == WDG_BOUNDARY ? 1 : 0,
+                               op->d_geom, op->d_nbr, op->d_info, op->d_basis, op->face_interp(),
+                               bnd ? op->n_bel : op->nel, bnd ? op->d_bel : nullptr, bnd ? 0 : 1, bnd ? 1 : 0,
                                as_stream(stream));
         hip_check(hipGetLastError(), "edge flux kernel launch");
     });
@@ -2072,7 +2056,8 @@ static int advection_launch(wdg_advection adv, const void* d_u, void* d_divF, bo
             wdg::launch_divf_linear(op->n, 0, a, s);
         }
         wdg::launch_advect_face(op->n, adv->nv, static_cast<const double*>(d_u), static_cast<double*>(d_divF),
-                                op->d_nbr, op->d_info, adv->d_H, op->face_interp(), op->nel, interior ? 1 : 0,
+                                op->d_nbr, op->d_info, adv->d_H, op->face_interp(),
+                                interior ? op->nel : op->n_bel, interior ? nullptr : op->d_bel, interior ? 1 : 0,
                                 boundary ? 1 : 0, s);
         hip_check(hipGetLastError(), "advection kernel launch");
     });

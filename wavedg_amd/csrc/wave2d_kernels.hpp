@@ -850,12 +850,19 @@ struct DivFArgs {
 };
 void launch_divf_linear(int n, int f32, const DivFArgs& a, hipStream_t s);
 
+// MassMatrix<true>: y = M x or M^{-1} x (inv) for nv variables per node, state
+// precision f32 or double, arithmetic in double (divf.hip); x may be y.
+void launch_mass(int n, int f32, const void* x, void* y, const double* corners, const double* basis, int nel, int nv,
+                 int inv, hipStream_t s);
+
 // Advection<true> / AdvectionHomogeneousBC<true> face terms (advect.hip):
 // y(node) += H_own u(node) + H_other u(neighbour node) for every node of the
 // selected sides, H per (element, side, node): (2, nv, nv) column-major.
 // P: face interpolation phi_m(-1) of a Gauss-Legendre basis, or null.
+// list: the nel elements to visit, or null for elements 0 .. nel - 1.
 void launch_advect_face(int n, int nv, const double* u, double* y, const int32_t* nbr, const int32_t* info,
-                        const double* H, const double* P, int nel, int interior, int boundary, hipStream_t s);
+                        const double* H, const double* P, int nel, const int32_t* list, int interior, int boundary,
+                        hipStream_t s);
 // Both terms of Advection<true>::action in one kernel, for up to three
 // variables (false: not covered; two kernels do it).  a as for
 // launch_divf_linear, H as for launch_advect_face.
@@ -876,8 +883,8 @@ void launch_advect_q(int n, int nv, int nq_volume, int nq_edge, const double* u,
 // y -= w ds LLF(n, q_own, q_other) at every node of the selected sides for the
 // compressible Euler flux (advect.hip); boundary sides take q_other = q_own.
 void launch_euler_face(int n, double gamma, const double* q, double* y, const double* geom, const int32_t* nbr,
-                       const int32_t* info, const double* basis, const double* P, int nel, int interior, int boundary,
-                       hipStream_t s);
+                       const int32_t* info, const double* basis, const double* P, int nel, const int32_t* list,
+                       int interior, int boundary, hipStream_t s);
 
 // DivF2D<true> / EdgeFluxF2D<true> with flux functors compiled from source
 // at run time (flux_rtc.hip).  Kernels compile on first use; the functions
