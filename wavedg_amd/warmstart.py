@@ -99,13 +99,17 @@ class WarmStart:
         torch = self.torch
         if out is None:
             out = torch.empty((len(specs), self.M, self.M, IN_LD), dtype=torch.bfloat16, device="cuda")
-        for b, spec in enumerate(specs):
-            src = np.asarray(spec["sources"], dtype=np.float64).reshape(-1, 4)
-            sd = torch.tensor(src.reshape(-1), device="cuda")
+        # one upload for all problems: a blocking copy per problem cost more
+        # than the problem's kernel
+        srcs = [np.asarray(spec["sources"], dtype=np.float64).reshape(-1, 4) for spec in specs]
+        sd = torch.tensor(np.concatenate([src.reshape(-1) for src in srcs]) if srcs else np.zeros(0), device="cuda")
+        stream, at = capi.cur_stream(), 0
+        for b, (spec, src) in enumerate(zip(specs, srcs)):
             s = source_scale(src)
-            capi.ws_features(self.nodes, self.n, self.nel, sd, src.shape[0], (1.0 / self.M) ** 2 / s, spec["omega"],
-                             omega_feature(spec["omega"]), 1.0 / s if self.green else 0.0, (0.0, 0.0, 1.0, 1.0),
-                             IN_LD, out[b])
+            capi.ws_features(self.nodes, self.n, self.nel, sd[at:at + src.size], src.shape[0], (1.0 / self.M) ** 2 / s,
+                             spec["omega"], omega_feature(spec["omega"]), 1.0 / s if self.green else 0.0,
+                             (0.0, 0.0, 1.0, 1.0), IN_LD, out[b], stream=stream)
+            at += src.size
         return out
 
     def targets(self, Ws, specs, out=None):
