@@ -279,8 +279,8 @@ struct NodeResult {
 // converting in the kernel, so results do not change).  LEG: Gauss-Legendre
 // basis, whose side traces interpolate along the element (inward_stride) and
 // whose face contributions lift back with the same weights P.
-template <int N, typename R, bool VOL, bool IFACE, bool BFACE, int TGT = 256, bool LEG = false, typename GT = double,
-          typename BT = double, typename Prefetch>
+template <int N, typename R, bool VOL, bool IFACE, bool BFACE, int TGT = 256, bool LEG = false, bool INB = false,
+          typename GT = double, typename BT = double, typename Prefetch>
 __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_in, const GT* __restrict__ geom,
                                                         const FaceGeom<R>* __restrict__ fgeo,
                                                         const FaceNb* __restrict__ fnb,
@@ -353,6 +353,11 @@ __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_
     // on the table (3 % faster at P = 7 in FP64).
     constexpr bool FTAB = N >= 6 && sizeof(R) == 4;
     FaceGeom<R> fgv[FP];
+    // INB: a neighbour in this workgroup has its trace read from the state tile
+    // after the barrier instead of from memory (at its offset from the tile's
+    // first value).
+    const int blk0 = 3 * NN * e0;
+    auto in_block = [&](int x) { return INB && (unsigned)(x - blk0) < (unsigned)cnt; };
     if constexpr (FACE) {
 #pragma unroll
         for (int p = 0; p < FP; ++p) {
@@ -364,7 +369,7 @@ __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_
             fnb3[p] = fx.x;
             finfo[p] = fx.y;
             nbv[p][0] = nbv[p][1] = nbv[p][2] = (R)0;
-            if (IFACE && fon && fx.x >= 0) {
+            if (IFACE && fon && fx.x >= 0 && !in_block(fx.x)) {
                 const R* q = u_in + (fx.x + k * (fx.y >> 16));
                 if constexpr (LEG) {
                     const int st = 3 * inward_stride<N>(fx.y & 3);
@@ -477,7 +482,24 @@ __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_
                     vA = s_u[el * 3 * NN + 3 * ln + 2];
                 }
                 R pB, uB, vB;
-                if (interior) {
+                if (interior && in_block(fnb3[pp])) {
+                    const R* q = s_u + (fnb3[pp] - blk0) + k * (inf >> 16);
+                    if constexpr (LEG) {
+                        pB = uB = vB = (R)0;
+                        const int st = 3 * inward_stride<N>(inf & 3);
+#pragma unroll
+                        for (int m = 0; m < N; ++m) {
+                            const R Pm = (R)s_P[m];
+                            pB = fma(Pm, q[m * st + 0], pB);
+                            uB = fma(Pm, q[m * st + 1], uB);
+                            vB = fma(Pm, q[m * st + 2], vB);
+                        }
+                    } else {
+                        pB = q[0];
+                        uB = q[1];
+                        vB = q[2];
+                    }
+                } else if (interior) {
                     pB = nbv[pp][0];
                     uB = nbv[pp][1];
                     vB = nbv[pp][2];
@@ -576,6 +598,12 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
     constexpr bool READ_DU = OUT == M_OUT_STAGE;
     constexpr bool LEG = (MODE & M_LEG) != 0;
     constexpr bool NT = (MODE & M_NT) != 0;
+    // Streaming stages read the traces of neighbours in the workgroup (most of
+    // those along a row of elements) from LDS: fewer cache requests beside the
+    // streams (512^2 P = 7 FP64 299 -> 279 us, 701 x 499 P = 5 FP32 129 -> 121,
+    // 301 x 257 P = 6 Gauss-Legendre 107 -> 101).  Stages that fit the cache are
+    // 0-4 % slower with it (the longer way from the barrier to the fluxes).
+    constexpr bool INB = NT;
     using L = OpLds<N, R, VOL, IFACE || BFACE, TGT, LEG>;
     __shared__ __align__(16) unsigned char lds[L::bytes];
 
@@ -629,11 +657,11 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
     constexpr bool F32 = std::is_same<R, float>::value;
     const FaceGeom<R>* fgeo = static_cast<const FaceGeom<R>*>(a.fgeo);
     if constexpr (F32)
-        q = apply_operator<N, R, VOL, IFACE, BFACE, TGT, LEG>(static_cast<const R*>(a.u_in), a.geom32, fgeo, a.fnb,
+        q = apply_operator<N, R, VOL, IFACE, BFACE, TGT, LEG, INB>(static_cast<const R*>(a.u_in), a.geom32, fgeo, a.fnb,
                                                          a.basis32, a.ha32, a.hb32, e0, nloc, lds, el, gb, g, active,
                                                          prefetch);
     else
-        q = apply_operator<N, R, VOL, IFACE, BFACE, TGT, LEG>(static_cast<const R*>(a.u_in), a.geom, fgeo, a.fnb,
+        q = apply_operator<N, R, VOL, IFACE, BFACE, TGT, LEG, INB>(static_cast<const R*>(a.u_in), a.geom, fgeo, a.fnb,
                                                          a.basis, (R)a.ha, (R)a.hb, e0, nloc, lds, el, gb, g, active,
                                                          prefetch);
     // FP64 stage outputs with streaming stores at orders whose elements do not
