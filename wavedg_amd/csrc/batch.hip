@@ -114,7 +114,13 @@ __device__ __forceinline__ void batch_body(const BatchArgs& a, const BatchBlock&
 
     R pre0 = 0, pre1 = 0, pre2 = 0, f0 = 0, f1 = 0, f2 = 0;
     double ac0 = 0, ac1 = 0, ac2 = 0, x0 = 0, x1 = 0, x2 = 0;
+    // the step's coefficients, requested with the state: dt is stored after
+    // the filter coefficients; -sin(omega t)/omega scales the forcing (WaveHoltz.cpp:65)
+    double dtv = 0, fsv = 0, cv = 0;
     auto prefetch = [&](bool act, size_t gb, uint32_t g) {
+        dtv = a.ctab[pr.coff + pr.nt + 1];
+        if (forced) fsv = a.ftab[pr.foff + 5 * (long long)s + st];
+        if constexpr (KIND == 2) cv = a.ctab[pr.coff + s + 1];
         if (!act) return;
         if constexpr (KIND != 0) {
             const R* dub = du + gb;
@@ -155,7 +161,7 @@ __device__ __forceinline__ void batch_body(const BatchArgs& a, const BatchBlock&
     if (active) {
         R r0 = q.r0, r1 = q.r1, r2 = q.r2;
         if (forced) {
-            const R fs = (R)a.ftab[pr.foff + 5 * (long long)s + st];  // -sin(omega t)/omega (WaveHoltz.cpp:65)
+            const R fs = (R)fsv;
             r0 += f0 * fs;
             r1 += f1 * fs;
             r2 += f2 * fs;
@@ -164,7 +170,7 @@ __device__ __forceinline__ void batch_body(const BatchArgs& a, const BatchBlock&
         r0 *= im;
         r1 *= im;
         r2 *= im;
-        const R dt = (R)a.ctab[pr.coff + pr.nt + 1];  // dt is stored after the coefficients
+        const R dt = (R)dtv;
         const R rb = (R)a.rk_b;
         R d0, d1, d2;
         if constexpr (KIND == 0) {
@@ -190,7 +196,7 @@ __device__ __forceinline__ void batch_body(const BatchArgs& a, const BatchBlock&
             u_out[g + 1] = w1;
             u_out[g + 2] = w2;
         } else {
-            const double c = a.ctab[pr.coff + s + 1];
+            const double c = cv;
             const double n0 = ac0 + c * (double)w0, n1 = ac1 + c * (double)w1, n2 = ac2 + c * (double)w2;
             double* ac = a.acc + pr.soff + gb;
             if (!period_end) {
