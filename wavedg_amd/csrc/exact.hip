@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64) void exact_face_kernel(const KArgs a, const Exa
 {
     constexpr int NN = N * N;
     __shared__ double s_out[3 * NN], s_A[3 * N], s_B[3 * N], s_c[3 * kQMax], s_P[kQMax * N], s_w[kQMax];
-    const int e = blockIdx.x, tid = threadIdx.x, nq = t.nqe;
+    const int e = a.list ? a.list[blockIdx.x] : (int)blockIdx.x, tid = threadIdx.x, nq = t.nqe;
     const double* u = static_cast<const double*>(a.u_in);
     for (int k = tid; k < 3 * NN; k += 64) s_out[k] = 0.0;
     for (int k = tid; k < nq * N; k += 64) s_P[k] = t.Pe[k];
@@ -754,7 +754,10 @@ void launch_all(int what, const KArgs& a, const ExactTables& t, const ExactMassT
     const dim3 grid(a.nel);
     switch (what) {
     case 0: hipLaunchKernelGGL(exact_volume_kernel<N>, grid, dim3(kBlk), 0, s, a, t, p0); break;
-    case 1: hipLaunchKernelGGL(exact_face_kernel<N>, grid, dim3(64), 0, s, a, t, p0, p1); break;
+    case 1:
+        if (!a.list || a.nlist > 0)
+            hipLaunchKernelGGL(exact_face_kernel<N>, a.list ? dim3(a.nlist) : grid, dim3(64), 0, s, a, t, p0, p1);
+        break;
     default: hipLaunchKernelGGL(exact_mass_kernel<N>, grid, dim3(kBlk), 0, s, a, r, m, p0, p1); break;
     }
 }

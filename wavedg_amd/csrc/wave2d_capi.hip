@@ -136,6 +136,8 @@ struct wdg_wave2d_s {
     int32_t* d_info = nullptr;
     int32_t* d_bel = nullptr;  // the elements with a boundary side
     int n_bel = 0;
+    int32_t* d_bblk = nullptr;  // the workgroups of the collocated kernels that hold one of them
+    int n_bblk = 0;
     std::map<int, double*> d_lftab;  // LinearFunctional tables per rule size (wdg_hip_linear_functional)
     void* d_fgeo = nullptr;      // FaceGeom<R> per element side (handle precision)
     wdg::FaceNb* d_fnb = nullptr;       // neighbour trace base and flags per element side
@@ -186,6 +188,7 @@ struct wdg_wave2d_s {
         dfree(d_nbr);
         dfree(d_info);
         dfree(d_bel);
+        dfree(d_bblk);
         dfree(d_fgeo);
         dfree(d_fnb);
         for (auto& kv : d_lftab) dfree(kv.second);
@@ -289,7 +292,14 @@ void launch_wave(int n, int kid, int f32, int sched, const KArgs& a, hipStream_t
 void apply_op(wdg_wave2d op, int kid, const KArgs& a, hipStream_t s)
 {
     if (!op->exact) {
-        launch_wave(op->n, kid, op->prec == WDG_F32, op->sched, a, s);
+        if (kid == wdg::K_BC) {
+            KArgs b = a;
+            b.list = op->d_bblk;
+            b.nlist = op->n_bblk;
+            launch_wave(op->n, kid, op->prec == WDG_F32, op->sched, b, s);
+        } else {
+            launch_wave(op->n, kid, op->prec == WDG_F32, op->sched, a, s);
+        }
         return;
     }
     const wdg::ExactTables t = op->tables();
@@ -297,7 +307,10 @@ void apply_op(wdg_wave2d op, int kid, const KArgs& a, hipStream_t s)
         wdg::launch_exact_volume(op->n, a, t, 1, s);
         wdg::launch_exact_face(op->n, a, t, 1, 0, s);
     } else if (kid == wdg::K_BC) {
-        wdg::launch_exact_face(op->n, a, t, 0, 1, s);
+        KArgs b = a;
+        b.list = op->d_bel;
+        b.nlist = op->n_bel;
+        wdg::launch_exact_face(op->n, b, t, 0, 1, s);
     } else if (op->exact_fused() && op->leg) {
         // The nodes of a Gauss-Legendre basis are the points of the default
         // volume rule, and every integrand of the operator has a degree that
@@ -894,6 +907,14 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
             op->d_bel = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * std::max<size_t>(bel.size(), 1)));
             hip_check(hipMemcpy(op->d_bel, bel.data(), sizeof(int32_t) * bel.size(), hipMemcpyHostToDevice),
                       "upload boundary elements");
+            const int epb = std::max(1, 256 / (n * n));  // wdg::Shape<N>::EPB
+            std::vector<int32_t> blk;
+            for (int32_t e : bel)
+                if (blk.empty() || blk.back() != e / epb) blk.push_back(e / epb);
+            op->n_bblk = (int)blk.size();
+            op->d_bblk = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * std::max<size_t>(blk.size(), 1)));
+            hip_check(hipMemcpy(op->d_bblk, blk.data(), sizeof(int32_t) * blk.size(), hipMemcpyHostToDevice),
+                      "upload boundary workgroups");
         }
         hip_check(hipMemcpy(op->d_basis, basis.data(), sizeof(double) * basis.size(), hipMemcpyHostToDevice),
                   "upload basis");

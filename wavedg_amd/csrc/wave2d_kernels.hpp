@@ -54,6 +54,8 @@ struct KArgs {
     const FaceNb* fnb;      // (4, nel) neighbour trace base and flags (build_face_tables)
     float ha32, hb32, dt32, rk_a32, rk_b32, fs32;  // the scalars above rounded to float (FP32 handles)
     uint32_t sr_seed;       // FP32 stages: seed of the state update's stochastic rounding (sr_seed())
+    const int32_t* list;    // boundary terms alone: the workgroups (collocated kernel) or elements (exact face
+    int nlist;              //   kernel) that have a boundary side; null: all
     int nt_store;           // 1: stage outputs as non-temporal stores (arrays beyond the Infinity Cache)
 };
 
@@ -607,15 +609,16 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
     using L = OpLds<N, R, VOL, IFACE || BFACE, TGT, LEG>;
     __shared__ __align__(16) unsigned char lds[L::bytes];
 
-    const int e0 = xcd_block(blockIdx.x, gridDim.x) * EPB;
+    // boundary terms alone (WaveBC::action) visit the listed workgroups: the
+    // others add nothing, and 7,500 of them that look and leave took 6.7 us at
+    // 331 x 227 P = 4, the 314 listed ones take 4.9
+    int blk;
+    if constexpr (BFACE && !VOL && !IFACE)
+        blk = a.list[blockIdx.x];
+    else
+        blk = xcd_block(blockIdx.x, gridDim.x);
+    const int e0 = blk * EPB;
     const int nloc = min(EPB, a.nel - e0);
-    if constexpr (BFACE && !VOL && !IFACE) {
-        // boundary terms alone (WaveBC::action): a workgroup whose elements
-        // have no boundary side adds nothing, so it leaves y untouched
-        const int t = threadIdx.x;
-        const bool bnd = t < 4 * nloc && a.nbr[4 * (size_t)e0 + t] < 0;
-        if (!__syncthreads_or(bnd)) return;
-    }
 
     // RK register / output / forcing / accumulator values, loaded early
     R pre0 = 0, pre1 = 0, pre2 = 0, fv0 = 0, fv1 = 0, fv2 = 0;

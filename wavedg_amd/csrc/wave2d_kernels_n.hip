@@ -66,7 +66,8 @@ void launch_legendre(int kid, int sched, const KArgs& a, hipStream_t s)
         }
     default: break;
     }
-    const int nblk = (a.nel + Shape<N>::EPB - 1) / Shape<N>::EPB;
+    const int nblk = kid == K_BC ? a.nlist : (a.nel + Shape<N>::EPB - 1) / Shape<N>::EPB;
+    if (nblk <= 0) return;
     const dim3 grid(nblk), block(Shape<N>::NT);
     switch (kid) {
 #define WDG_CASE(K)                                                                      \
@@ -106,7 +107,8 @@ void launch_typed(int kid, int sched, const KArgs& a, hipStream_t s)
         }
     default: break;
     }
-    const int nblk = (a.nel + Shape<N>::EPB - 1) / Shape<N>::EPB;
+    const int nblk = kid == K_BC ? a.nlist : (a.nel + Shape<N>::EPB - 1) / Shape<N>::EPB;
+    if (nblk <= 0) return;
     const dim3 grid(nblk), block(Shape<N>::NT);
     switch (kid) {
 #define WDG_CASE(K)                                                              \
