@@ -134,7 +134,7 @@ struct wdg_wave2d_s {
     float* d_basis32 = nullptr;
     int32_t* d_nbr = nullptr;
     int32_t* d_info = nullptr;
-    int32_t* d_bel = nullptr;  // the elements with a boundary side
+    int32_t* d_bel = nullptr;   // the elements with a boundary side (behind d_info's words)
     int n_bel = 0;
     int32_t* d_bblk = nullptr;  // the workgroups of the collocated kernels that hold one of them
     int n_bblk = 0;
@@ -187,8 +187,6 @@ struct wdg_wave2d_s {
         dfree(d_basis32);
         dfree(d_nbr);
         dfree(d_info);
-        dfree(d_bel);
-        dfree(d_bblk);
         dfree(d_fgeo);
         dfree(d_fnb);
         for (auto& kv : d_lftab) dfree(kv.second);
@@ -886,7 +884,25 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
                   "upload geometry");
         op->d_corners = static_cast<double*>(dmalloc(sizeof(double) * m.corners().size()));
         op->d_nbr = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * ft.nbr.size()));
+        // the elements with a boundary side, then the workgroups of the collocated
+        // kernels that hold one, ride behind the info words in one array
+        {
+            const int epb = std::max(1, 256 / (n * n));  // wdg::Shape<N>::EPB
+            std::vector<int32_t> blk;
+            const size_t ni = ft.info.size();
+            for (int e = 0; e < op->nel; ++e) {
+                const int32_t* nb = &ft.nbr[4 * (size_t)e];
+                if ((nb[0] | nb[1] | nb[2] | nb[3]) >= 0) continue;  // no side is -1
+                ft.info.push_back(e);
+                if (blk.empty() || blk.back() != e / epb) blk.push_back(e / epb);
+            }
+            op->n_bel = (int)(ft.info.size() - ni);
+            op->n_bblk = (int)blk.size();
+            ft.info.insert(ft.info.end(), blk.begin(), blk.end());
+        }
         op->d_info = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * ft.info.size()));
+        op->d_bel = op->d_info + 4 * (size_t)op->nel;
+        op->d_bblk = op->d_bel + op->n_bel;
         op->d_basis = static_cast<double*>(dmalloc(sizeof(double) * basis.size()));
         op->d_lvtab = static_cast<double*>(dmalloc(sizeof(double) * lv.size()));
         op->d_partial = static_cast<double*>(dmalloc(sizeof(double) * kRedBlocks));
@@ -897,25 +913,6 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
                   "upload nbr");
         hip_check(hipMemcpy(op->d_info, ft.info.data(), sizeof(int32_t) * ft.info.size(), hipMemcpyHostToDevice),
                   "upload info");
-        {
-            std::vector<int32_t> bel;
-            for (int e = 0; e < op->nel; ++e)
-                if (ft.nbr[4 * (size_t)e] < 0 || ft.nbr[4 * (size_t)e + 1] < 0 || ft.nbr[4 * (size_t)e + 2] < 0 ||
-                    ft.nbr[4 * (size_t)e + 3] < 0)
-                    bel.push_back(e);
-            op->n_bel = (int)bel.size();
-            op->d_bel = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * std::max<size_t>(bel.size(), 1)));
-            hip_check(hipMemcpy(op->d_bel, bel.data(), sizeof(int32_t) * bel.size(), hipMemcpyHostToDevice),
-                      "upload boundary elements");
-            const int epb = std::max(1, 256 / (n * n));  // wdg::Shape<N>::EPB
-            std::vector<int32_t> blk;
-            for (int32_t e : bel)
-                if (blk.empty() || blk.back() != e / epb) blk.push_back(e / epb);
-            op->n_bblk = (int)blk.size();
-            op->d_bblk = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * std::max<size_t>(blk.size(), 1)));
-            hip_check(hipMemcpy(op->d_bblk, blk.data(), sizeof(int32_t) * blk.size(), hipMemcpyHostToDevice),
-                      "upload boundary workgroups");
-        }
         hip_check(hipMemcpy(op->d_basis, basis.data(), sizeof(double) * basis.size(), hipMemcpyHostToDevice),
                   "upload basis");
         hip_check(hipMemcpy(op->d_lvtab, lv.data(), sizeof(double) * lv.size(), hipMemcpyHostToDevice),
