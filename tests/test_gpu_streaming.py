@@ -1,8 +1,8 @@
 """Stage kernels with streaming (non-temporal) stores, which a handle selects
 when its three stage arrays exceed the 256 MiB Infinity Cache.  In FP64 the
 stage outputs then leave through LDS: at n = 8 each wavefront stages its
-element's block, at other orders the workgroup stages its block when
-EPB * 3 n^2 is even (otherwise the lanes store their own values).
+element's block, at other orders the workgroup stages its block, in 16-byte
+pieces when EPB * 3 n^2 is even and in single values otherwise.
 
 * RK4 steps on meshes above the threshold, at odd and even orders, on
   Gauss-Lobatto and Gauss-Legendre bases, under every workgroup schedule (so
