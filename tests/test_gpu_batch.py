@@ -163,3 +163,25 @@ def test_batch_replay_length_changes_nothing(cuda, precision):
             ref = got
         for (i0, r0, W0), (i1, r1, W1) in zip(ref, got):
             assert i0 == i1 and r0 == r1 and torch.equal(W0, W1)
+
+
+@pytest.mark.parametrize("count", [1, 5], ids=["runs", "in-turn"])
+def test_batch_workgroup_order_changes_nothing(cuda, count):
+    """Stage arrays below the Infinity Cache's 256 MB (one problem, 68 MB) and
+    above it (five, 340 MB) take the two orders of the workgroups; 95^2
+    elements leave the last workgroup and the XCDs' runs uneven."""
+    torch = cuda
+    v, e = meshgen.uniform_rect(95, 0.0, 1.0, 95, 0.0, 1.0)
+    m = capi.Mesh(v, e)
+    probs = [dict(mesh=m, n=8, omega=95.0 * 64 * 4.0 * np.pi / 200, sources=[[0.3 + 0.05 * k, 0.4, 0.08, 1.0]],
+                  bc=bc_codes(m.n_boundary, "mixed", seed=k)) for k in range(count)]
+    b = capi.Batch(probs)
+    print(f"batch of {count}, periods {[b.info(k)[1] for k in range(count)]}", flush=True)
+    b.solve(1e-14, 2, steps_per_graph=8)
+    for k, pb in enumerate(probs):
+        Ws, its, rs, _ = _solo(torch, pb, 1e-14, 2)
+        Wb = torch.empty_like(Ws)
+        itb, rb = b.result(k, Wb)
+        torch.cuda.synchronize()
+        assert itb == its and abs(rb - rs) <= 1e-9 * rs
+        assert rel_l2(Wb.cpu().numpy(), Ws.cpu().numpy()) < 1e-12

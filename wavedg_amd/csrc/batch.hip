@@ -80,6 +80,7 @@ struct BatchArgs {
     int stage;
     int step;        // this launch's step after *G
     int check;       // 1: problems may retire between the launches of one replay
+    int runs;        // 1: one contiguous run of workgroups per XCD
 };
 
 constexpr int kBT = 256;  // threads per workgroup
@@ -256,9 +257,9 @@ template <typename R, int KIND>
 __global__ __launch_bounds__(kBT) void batch_stage_kernel(const BatchArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds[];
-    // each XCD walks one contiguous run of workgroups, so that neighbouring
-    // elements of a problem share its L2
-    const BatchBlock blk = a.blocks[wdg::xcd_block(blockIdx.x, gridDim.x)];
+    // with `runs`, each XCD walks one contiguous run of workgroups, so that
+    // neighbouring elements of a problem share its L2
+    const BatchBlock blk = a.blocks[a.runs ? wdg::xcd_block(blockIdx.x, gridDim.x) : blockIdx.x];
     if (a.check && !a.active[blk.prob]) return;  // uniform per workgroup
     const BatchProb& pr = blk.pr;
     const long long G = *a.G + a.step;
@@ -432,6 +433,7 @@ struct wdg_batch_s {
     long long ntot = 0;  // total state length
     std::vector<BatchProb> probs;
     std::vector<BatchBlock> all_blocks;  // full workgroup table
+    bool xcd_runs = true;  // compact(): one run of workgroups per XCD
     int n_run_blocks = 0, n_run_probs = 0;  // compacted tables of the problems still running
     int* d_prob_ids = nullptr;
     std::vector<long long> ndof;
@@ -506,6 +508,7 @@ struct wdg_batch_s {
         a.rk_a = kA[stage];
         a.rk_b = kB[stage];
         a.stage = stage;
+        a.runs = xcd_runs ? 1 : 0;
         return a;
     }
 };
@@ -547,6 +550,16 @@ void compact(wdg_batch_s& b, const std::vector<int>& run, hipStream_t s)
     }
     b.n_run_blocks = (int)blocks.size();
     b.n_run_probs = (int)ids.size();
+    // Runs per XCD while the arrays of a stage (two states, du, the forcing and
+    // the FP64 filter sum) fit the 256 MB Infinity Cache: there L2 hits decide
+    // (one period of 2 problems of 128^2 at P = 4, 98 MB: 56.0 ms against 60.4
+    // dealt in turn; of 5, 246 MB: 117.8 against 127.3).  Beyond it HBM does, which
+    // one compact window of addresses serves better than eight distant ones
+    // (4 of 96^2 at P = 7, 283 MB: 143.6 dealt against 150.7; 8 of 200^2 at
+    // P = 6, 1.4 GB: 1221 against 1269; FP32 12 of 128^2, 354 MB: 211.7 against 218.0).
+    double dofs = 0;
+    for (int k : ids) dofs += 3.0 * b.probs[k].nel * b.probs[k].N * b.probs[k].N;
+    b.xcd_runs = (4.0 * b.rsz + 8.0) * dofs <= 268435456.0;
     if (blocks.empty()) return;
     bcheck(hipMemcpyAsync(b.d_blocks, blocks.data(), sizeof(BatchBlock) * blocks.size(), hipMemcpyHostToDevice, s),
            "upload blocks");
