@@ -1177,7 +1177,12 @@ int wdg_hip_rk4_steps(wdg_wave2d op, double dt, double* t, void* d_u, int n_step
         void* third = nullptr;
         if (n_steps & 1) {
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
+            // HIP refuses this query on the null stream while a blocking stream
+            // of the process captures; the steps themselves run there
+            if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+                (void)hipGetLastError();
+                cap = hipStreamCaptureStatusActive;
+            }
             if (!op->d_r1 && cap == hipStreamCaptureStatusNone) {
                 std::lock_guard<std::mutex> lk(wdg::capture_mutex());
                 if (hipMalloc(&op->d_r1, op->state_bytes()) != hipSuccess) {
