@@ -278,7 +278,10 @@ int wdg_hip_wave2d_rhs(wdg_wave2d op, const void *d_x, void *d_y, const void *d_
 /* n_steps of ode::RungeKutta4::step (ode.hpp:66-93) on u' = M^{-1}(A+B)u
  * [- F sin(omega t)/omega if d_F != NULL and omega > 0, as in WaveHoltz::pi0],
  * each stage one fused kernel.  *t is advanced by n_steps dt.  d_u is updated
- * in place; d_F has the handle's precision. */
+ * in place; d_F has the handle's precision.  The handle keeps two state-sized
+ * buffers from the first call on, and from its second call with an odd n_steps
+ * a third one where that is at most a sixteenth of the free device memory
+ * (without it the result is copied back to d_u). */
 int wdg_hip_rk4_steps(wdg_wave2d op, double dt, double *t, void *d_u, int n_steps, const void *d_F, double omega,
                       void *stream);
 /* Same as wdg_hip_rk4_steps with d_F = NULL, captured once into a HIP graph

@@ -145,8 +145,10 @@ struct wdg_wave2d_s {
     double* d_lvtab = nullptr;
     void* d_tmp = nullptr;  // RK ping-pong partner of the caller's state
     void* d_du = nullptr;   // RK register
-    void* d_r1 = nullptr;   // scratch state-sized buffers (postprocess, conversions)
+    void* d_r1 = nullptr;   // scratch state-sized buffers (postprocess, conversions, odd numbers of steps)
     void* d_r2 = nullptr;
+    int odd_calls = 0;         // odd_step_buffer(): calls so far without a buffer,
+    bool third_asked = false;  //   and whether it has been asked for
     double* d_partial = nullptr;
     double* d_result = nullptr;
     bool timing = false;
@@ -494,6 +496,37 @@ void* run_steps(wdg_wave2d op, double dt, double& t, void* u, int n_steps, const
         t += dt;
     }
     return cur;
+}
+
+// Where an odd number of steps ends.  Its last stage writes the ping-pong
+// partner of the caller's array, so either the result is copied back or the
+// first three stages go round through a third state-sized buffer: two words
+// per unknown less (states of 250 MB at P = 7: one step 1017 -> 914 us, three
+// 2752 -> 2676 us; of 10 MB 61.5 -> 55.0 us).  Returns that buffer, or null for
+// the copy.  A program that makes one odd call neither waits for the
+// allocation nor holds the memory: the buffer comes with the second such call.
+// It is asked for once and only where it is at most a sixteenth of the free
+// device memory, so that what the handle keeps does not starve the caller.
+void* odd_step_buffer(wdg_wave2d op, hipStream_t s)
+{
+    if (op->d_r1 || op->third_asked || ++op->odd_calls < 2) return op->d_r1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    // HIP refuses this query on the null stream while a blocking stream of the
+    // process captures; the steps themselves run there
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    op->third_asked = true;
+    std::lock_guard<std::mutex> lk(wdg::capture_mutex());
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || op->state_bytes() > free_bytes / 16 ||
+        hipMalloc(&op->d_r1, op->state_bytes()) != hipSuccess) {
+        (void)hipGetLastError();
+        op->d_r1 = nullptr;
+    }
+    return op->d_r1;
 }
 
 struct NoCoef {
@@ -1171,27 +1204,7 @@ int wdg_hip_rk4_steps(wdg_wave2d op, double dt, double* t, void* d_u, int n_step
         const hipStream_t s = as_stream(stream);
         start_timing(op, s);
         double tt = *t;
-        // An odd number of steps ends in the ping-pong partner: a third buffer
-        // instead of a copy back (two of 19 words per unknown for one step; 3
-        // steps of 701 x 499 P = 5 in FP32 1910 -> 1858 us), where it can be had.
-        void* third = nullptr;
-        if (n_steps & 1) {
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            // HIP refuses this query on the null stream while a blocking stream
-            // of the process captures; the steps themselves run there
-            if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-                (void)hipGetLastError();
-                cap = hipStreamCaptureStatusActive;
-            }
-            if (!op->d_r1 && cap == hipStreamCaptureStatusNone) {
-                std::lock_guard<std::mutex> lk(wdg::capture_mutex());
-                if (hipMalloc(&op->d_r1, op->state_bytes()) != hipSuccess) {
-                    (void)hipGetLastError();
-                    op->d_r1 = nullptr;
-                }
-            }
-            third = op->d_r1;
-        }
+        void* third = n_steps & 1 ? odd_step_buffer(op, s) : nullptr;
         void* fin = run_steps(op, dt, tt, d_u, n_steps, d_F, omega, nullptr, NoCoef{}, s, third);
         stop_timing(op, s, 5 * n_steps);
         if (fin != d_u)
