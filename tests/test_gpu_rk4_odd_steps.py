@@ -25,16 +25,18 @@ def _wave(v, e, n):
 
 @pytest.mark.parametrize("flags", [BLOCKING, NON_BLOCKING])
 @pytest.mark.parametrize("mode", [0, 1, 2])  # global, thread-local, relaxed
-def test_null_stream_steps_beside_a_capture(cuda, flags, mode):
+@pytest.mark.parametrize("before", [1, 2])
+def test_null_stream_steps_beside_a_capture(cuda, flags, mode, before):
     """While a blocking stream captures, HIP refuses to say whether the null
-    stream does; launches on the null stream run all the same."""
+    stream does; launches on the null stream run all the same.  With one odd
+    call before, this call is the one that asks for the third buffer."""
     torch = cuda
     assert torch.cuda.current_stream().cuda_stream == 0
     hip = ctypes.CDLL("libamdhip64.so")
     w, dt = _wave(*mesh_case("skewed6x5"), 4)
     u0 = torch.tensor(random_state(w.ndof, 3), device="cuda")
     ref = u0.clone()
-    for _ in range(2):  # scratch in place before the capture
+    for _ in range(before):
         ref.copy_(u0)
         w.rk4(ref, dt, 3)
     s, g = ctypes.c_void_p(), ctypes.c_void_p()

@@ -520,12 +520,17 @@ void* odd_step_buffer(wdg_wave2d op, hipStream_t s)
     if (cap != hipStreamCaptureStatusNone) return nullptr;
     op->third_asked = true;
     std::lock_guard<std::mutex> lk(wdg::capture_mutex());
+    // an allocation in the thread's default capture mode would end a global
+    // capture of another stream
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hip_check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || op->state_bytes() > free_bytes / 16 ||
         hipMalloc(&op->d_r1, op->state_bytes()) != hipSuccess) {
         (void)hipGetLastError();
         op->d_r1 = nullptr;
     }
+    hip_check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
     return op->d_r1;
 }
 
