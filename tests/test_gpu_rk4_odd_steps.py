@@ -1,7 +1,7 @@
 """Odd numbers of fused RK4 steps, whose stages end in the ping-pong partner:
 the caller's array holds the result wherever the steps run, also on the null
 stream while another stream of the process captures, and what the handle
-keeps for them in device memory is bounded."""
+keeps for them in device memory is bounded and pays."""
 from __future__ import annotations
 
 import ctypes
@@ -84,6 +84,31 @@ def test_third_buffer_comes_with_the_second_odd_call(cuda):
     w.rk4(x, dt, 2)
     w.rk4(x, dt, 1)
     assert all(torch.equal(x, o) for o in outs)
+
+
+@pytest.mark.parametrize("precision,n,mb,buffer", [
+    (capi.F64, 8, 75, False), (capi.F64, 5, 70, False), (capi.F32, 8, 75, False), (capi.F32, 3, 80, True),
+    (capi.F64, 8, 60, True), (capi.F64, 8, 90, True)])
+def test_copy_where_only_three_states_fit_the_cache(cuda, precision, n, mb, buffer):
+    """States of 70-80 MB: three fit the 256 MB cache and four do not, unless
+    the tables of small elements (FP32, n = 3) fill it."""
+    torch = cuda
+    rsz = 4 if precision == capi.F32 else 8
+    nx = int((mb * 1e6 / (3 * n * n * rsz)) ** 0.5)
+    gm = capi.Mesh(*meshgen.uniform_rect(nx, 0.0, 1.0, nx, 0.0, 1.0))
+    w = capi.Wave2D(gm, n, np.ones(gm.n_boundary, dtype=np.int32), precision=precision)
+    dt = 0.4 * gm.min_h() / n**2
+    u0 = torch.tensor(random_state(w.ndof, 21), dtype=w.torch_dtype, device="cuda")
+    a, b = u0.clone(), u0.clone()
+    w.rk4(a, dt, 2)
+    w.rk4(a, dt, 1)
+    free = _free(torch)
+    w.rk4(b, dt, 1)
+    used = free - _free(torch)
+    assert used >= rsz * w.ndof if buffer else used == 0
+    a.copy_(u0)
+    w.rk4(a, dt, 1)
+    assert torch.equal(a, b)
 
 
 def test_third_buffer_stays_below_a_sixteenth_of_the_free_memory(cuda):

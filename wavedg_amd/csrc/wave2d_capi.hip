@@ -507,8 +507,21 @@ void* run_steps(wdg_wave2d op, double dt, double& t, void* u, int n_steps, const
 // allocation nor holds the memory: the buffer comes with the second such call.
 // It is asked for once and only where it is at most a sixteenth of the free
 // device memory, so that what the handle keeps does not starve the caller.
-void* odd_step_buffer(wdg_wave2d op, hipStream_t s)
+// The copy stays where a stage's three states and tables fit the 256 MB
+// Infinity Cache and a fourth state does not: the round through it then costs
+// misses (one step in FP64, buffer and copy: 75 MB states P = 4 325 and 300 us,
+// P = 7 296 and 278; 81 MB P = 5 363 and 343, P = 7 339 and 312).  Smaller
+// states gain from the buffer (50 MB, P = 7: 184 and 202), larger ones miss
+// either way (95 MB: 365 and 388).  Between 75 and 85 MB single handles differ
+// by up to 10 % with the addresses they get; the line is that of the mean.
+void* odd_step_buffer(wdg_wave2d op, bool forced, hipStream_t s)
 {
+    const double cache = 256.0 * 1024 * 1024, state = (double)op->state_bytes();
+    // per element: map coefficients, face neighbours, FP32 side normals where read
+    const double tables = (double)op->nel * (6.0 * op->rsz + 4.0 * sizeof(wdg::FaceNb) +
+                                             (op->prec == WDG_F32 && op->n >= 6 ? 4.0 * sizeof(wdg::FaceGeom<float>) : 0.0));
+    const double three = (forced ? 4.0 : 3.0) * state + tables;
+    if (three <= cache && three + state > cache) return nullptr;
     if (op->d_r1 || op->third_asked || ++op->odd_calls < 2) return op->d_r1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     // HIP refuses this query on the null stream while a blocking stream of the
@@ -1209,7 +1222,7 @@ int wdg_hip_rk4_steps(wdg_wave2d op, double dt, double* t, void* d_u, int n_step
         const hipStream_t s = as_stream(stream);
         start_timing(op, s);
         double tt = *t;
-        void* third = n_steps & 1 ? odd_step_buffer(op, s) : nullptr;
+        void* third = n_steps & 1 ? odd_step_buffer(op, d_F != nullptr, s) : nullptr;
         void* fin = run_steps(op, dt, tt, d_u, n_steps, d_F, omega, nullptr, NoCoef{}, s, third);
         stop_timing(op, s, 5 * n_steps);
         if (fin != d_u)
