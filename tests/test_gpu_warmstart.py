@@ -40,3 +40,19 @@ def test_warm_start_reduces_iterations(cuda, M, count):
     err = [float(torch.linalg.norm(p - b) / torch.linalg.norm(b)) for p, b in zip(pred, Wp)]
     print(f"prediction relative errors {np.round(err, 3)}", flush=True)
     assert np.median(err) < 0.2
+
+
+def test_features_walk_any_iterable(cuda):
+    """Problems given one by one (an iterator) into the caller's array, with
+    different numbers of sources, give each problem's own image."""
+    torch = cuda
+    ws = warmstart.WarmStart(16, max_batch=4)
+    src = [[0.3, 0.6, 0.02, 1.0], [0.7, 0.4, 0.01, -0.5], [0.5, 0.5, 0.03, 2.0]]
+    specs = [dict(omega=20.0 + 5.0 * k, sources=src[:k + 1]) for k in range(3)]
+    want = torch.cat([ws.features([sp]) for sp in specs])
+    shape = (3, 16, 16, warmstart.IN_LD)
+    for given in (specs, tuple(specs), iter(specs)):
+        out = torch.full(shape, -7.0, dtype=torch.bfloat16, device="cuda")
+        assert ws.features(given, out) is out
+        assert torch.equal(out, want)
+    assert tuple(ws.features([]).shape) == (0, 16, 16, warmstart.IN_LD)

@@ -101,6 +101,7 @@ class WarmStart:
             out = torch.empty((len(specs), self.M, self.M, IN_LD), dtype=torch.bfloat16, device="cuda")
         # one upload for all problems: a blocking copy per problem cost more
         # than the problem's kernel
+        specs = list(specs)  # any iterable where out is given; it is walked twice
         srcs = [np.asarray(spec["sources"], dtype=np.float64).reshape(-1, 4) for spec in specs]
         sd = torch.tensor(np.concatenate([src.reshape(-1) for src in srcs]) if srcs else np.zeros(0), device="cuda")
         stream, at = capi.cur_stream(), 0
