@@ -2301,11 +2301,12 @@ int wdg_hip_cnn_create(int M, int in_ld, int out_channels, int base_width, int m
             L.wb = foff;
             foff += nw;
             const int H = M >> L.level;
-            // the largest chunk count any batch size up to max_batch uses
+            // the largest chunk count any batch size up to max_batch uses (bwd()
+            // takes the row kernel for images at least 16 wide)
             long long tchunks = 0;
             for (int bb = 1; bb <= max_batch; ++bb)
-                tchunks = std::max<long long>({tchunks, wgrad_tiled_chunks(L, bb, H, nullptr),
-                                               wgrad_row_chunks(L, bb, H, nullptr)});
+                tchunks = std::max<long long>(
+                    tchunks, H >= 16 ? wgrad_row_chunks(L, bb, H, nullptr) : wgrad_tiled_chunks(L, bb, H, nullptr));
             const long long chunks =
                 std::max<long long>(((long long)max_batch * H * H + kChunk - 1) / kChunk, tchunks);
             const long long bchunks = ((long long)max_batch * H * H + kBiasChunk - 1) / kBiasChunk;
