@@ -143,15 +143,17 @@ def test_dg_image_maps(cuda):
     assert float(torch.linalg.norm(W2 - W) / torch.linalg.norm(W)) < 1e-7
 
 
-def test_convolution_tiles_agree(cuda):
-    """Every tile of conv3_row_kernel against the smallest one: a batch of 16
-    images of 128^2 runs the four levels on tiles of 512, 256, 128 and 64
-    pixels, one image alone on 64 everywhere.  The tiles add in the same order,
-    so outputs are equal bit for bit; the batch gradient is the mean of the
-    single ones up to the order of its float32 sums (the loss gradient is
-    scaled by 1/16, exactly)."""
+@pytest.mark.parametrize("M,B", [(128, 16), (32, 128), (32, 256)])
+def test_convolution_tiles_agree(cuda, M, B):
+    """Tiles of conv3_row_kernel against its smallest, which one image alone
+    takes everywhere.  16 images of 128^2 run the widths 128, 64, 32 and 16 on
+    512, 256, 128 and 64 pixels (backward-data also on 256 at width 32); 128
+    and 256 images of 32^2 reach the taller tiles of the widths 32 and 16: 512
+    at 32, 256 and 128 at 16.  The tiles add in the same order, so outputs are
+    equal bit for bit; the batch gradient is the mean of the single ones up to
+    the order of its float32 sums (the loss gradient is scaled by a power of
+    two, exactly)."""
     torch = cuda
-    M, B = 128, 16
     net, p, x, t, xd, td = _setup(torch, M=M, base=32, in_ld=48, B=B, seed=21)
     y = torch.empty((B, M, M, net.out_ld), dtype=torch.float32, device="cuda")
     net.forward(xd, y)
@@ -167,6 +169,30 @@ def test_convolution_tiles_agree(cuda):
     assert abs(loss - np.mean(losses)) < 1e-6 * loss
     # float32 partial sums over at most 2^18 pixels in chunks: below 2^-24 * 2^7
     assert _rel(g, mean) < 1e-5
+
+
+@pytest.mark.parametrize("M,base,B", [(128, 32, 9), (128, 64, 3), (64, 32, 13)])
+def test_weight_gradient_of_an_odd_number_of_strips(cuda, M, base, B):
+    """wgrad3_row_kernel<4, 16> takes two 16-pixel images per tile; an odd
+    batch leaves the last tile with one, whose missing partner reads as zeros.
+    The batch against itself twice over, which fills every tile: the mean loss
+    and so each layer's gradient are the same (the loss gradient is halved,
+    exactly) up to the order of the float32 sums, layer by layer."""
+    torch = cuda
+    H, L = 16, {128: 3, 64: 2}[M]
+    cin, cout = {3: (8 * base, 8 * base), 2: (12 * base, 4 * base)}[L]
+    assert M >> L == H and B % 2 == 1
+    assert B * H * H // 512 * (cout // 32) * (cin // 32) >= 256, "the rule must choose the taller tile"
+    net, p, x, t, xd, td = _setup(torch, M=M, base=base, in_ld=48, B=2 * B, seed=33)
+    x2, t2 = torch.cat([xd[:B], xd[:B]]), torch.cat([td[:B], td[:B]])
+    l1, g1 = net.loss_grad(xd[:B], td[:B])
+    l2, g2 = net.loss_grad(x2, t2)
+    assert abs(l1 - l2) < 1e-6 * l1
+    for name, wo, bo, shp in co.Net(p, net.in_ld, 75, base).layout:
+        sl = slice(wo, bo + shp[1])
+        err = _rel(g1[sl], g2[sl].astype(np.float64))
+        print(f"  {name}: {err:.2e}", flush=True)
+        assert err < 1e-5, name  # below 2^-24 * 2^7, as above
 
 
 def test_row_convolution_matches_oracle(cuda):

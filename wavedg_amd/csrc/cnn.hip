@@ -1906,7 +1906,7 @@ void launch_conv(const wdg_cnn_s& n, hipStream_t s, const uint16_t* in, int in_l
             launch_conv_row<r, nw, 4>(s, a, f32out);                                                            \
         else if (WX == 2)                                                                                       \
             launch_conv_row<r, nw, 2>(s, a, f32out);                                                            \
-        else                                                                                                    \
+        else if constexpr (r * nw <= 16) /* fits(): 16-pixel images have no taller tile */                     \
             launch_conv_row<r, nw, 1>(s, a, f32out);                                                            \
         return;                                                                                                 \
     }
