@@ -938,7 +938,7 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
         // the elements with a boundary side, then the workgroups of the collocated
         // kernels that hold one, ride behind the info words in one array
         {
-            const int epb = std::max(1, 256 / (n * n));  // wdg::Shape<N>::EPB
+            const int epb = wdg::elems_per_block(n);
             std::vector<int32_t> blk;
             const size_t ni = ft.info.size();
             for (int e = 0; e < op->nel; ++e) {

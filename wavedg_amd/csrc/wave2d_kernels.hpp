@@ -170,16 +170,21 @@ __device__ __forceinline__ void st_stream(T* p, T v)
 // Workgroup schedule: about TGT threads, i.e. EPB = TGT / n^2 whole elements
 // (at least one).  TGT = 64 at n = 8 is one wavefront per element; smaller
 // orders pack several elements into each wavefront.
-template <int N, int TGT = 256>
+constexpr int kTgt = 256;  // the schedule of every kernel that takes no other
+
+// Elements per workgroup; host code that lists workgroups asks here too.
+constexpr int elems_per_block(int n, int tgt = kTgt) { return tgt / (n * n) > 0 ? tgt / (n * n) : 1; }
+
+template <int N, int TGT = kTgt>
 struct Shape {
     static constexpr int NN = N * N;
-    static constexpr int EPB = (TGT / NN) > 0 ? (TGT / NN) : 1;  // elements per workgroup
+    static constexpr int EPB = elems_per_block(N, TGT);
     static constexpr int NT = EPB * NN;                          // threads per workgroup
 };
 
 // Schedules the stage kernels can be launched with (index -> TGT).
 constexpr int kSchedules = 4;
-constexpr int kSchedTgt[kSchedules] = {256, 512, 128, 64};
+constexpr int kSchedTgt[kSchedules] = {kTgt, 512, 128, 64};
 
 // Workgroups are dealt to the 8 XCDs round-robin (b -> XCD b mod 8).  Give
 // each XCD one contiguous run of elements so that an element's neighbours
@@ -243,7 +248,7 @@ __device__ __forceinline__ int inward_stride(int s)
 }
 
 // LDS carve-up of apply_operator for one workgroup of Shape<N, TGT> elements.
-template <int N, typename R, bool VOL, bool FACE, int TGT = 256, bool LEG = false>
+template <int N, typename R, bool VOL, bool FACE, int TGT = kTgt, bool LEG = false>
 struct OpLds {
     static constexpr int NN = N * N, EPB = Shape<N, TGT>::EPB, NF = 4 * N;
     static constexpr int NXW = LEG ? 3 * N : 2 * N;  // x[N], w[N] (, P[N])
@@ -281,7 +286,7 @@ struct NodeResult {
 // converting in the kernel, so results do not change).  LEG: Gauss-Legendre
 // basis, whose side traces interpolate along the element (inward_stride) and
 // whose face contributions lift back with the same weights P.
-template <int N, typename R, bool VOL, bool IFACE, bool BFACE, int TGT = 256, bool LEG = false, bool INB = false,
+template <int N, typename R, bool VOL, bool IFACE, bool BFACE, int TGT = kTgt, bool LEG = false, bool INB = false,
           typename GT = double, typename BT = double, typename Prefetch>
 __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_in, const GT* __restrict__ geom,
                                                         const FaceGeom<R>* __restrict__ fgeo,
@@ -586,7 +591,7 @@ __device__ __forceinline__ NodeResult<R> apply_operator(const R* __restrict__ u_
     return out;
 }
 
-template <int N, typename R, int MODE, int TGT = 256>
+template <int N, typename R, int MODE, int TGT = kTgt>
 __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVES_F32 : WDG_MIN_WAVES)) void wave_kernel(
     const KArgs a)
 {
