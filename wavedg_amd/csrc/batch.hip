@@ -556,7 +556,7 @@ void compact(wdg_batch_s& b, const std::vector<int>& run, hipStream_t s)
     // dealt in turn; of 5, 246 MB: 117.8 against 127.3).  Beyond it HBM does, which
     // one compact window of addresses serves better than eight distant ones
     // (4 of 96^2 at P = 7, 283 MB: 143.6 dealt against 150.7; 8 of 200^2 at
-    // P = 6, 1.4 GB: 1221 against 1269; FP32 12 of 128^2, 354 MB: 211.7 against 218.0).
+    // P = 6, 1.9 GB: 1221 against 1269; FP32 12 of 128^2, 354 MB: 211.7 against 218.0).
     double dofs = 0;
     for (int k : ids) dofs += 3.0 * b.probs[k].nel * b.probs[k].N * b.probs[k].N;
     b.xcd_runs = (4.0 * b.rsz + 8.0) * dofs <= 268435456.0;
