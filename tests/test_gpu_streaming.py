@@ -9,6 +9,9 @@ pieces when EPB * 3 n^2 is even and in single values otherwise.
   the staged and the per-lane store paths both run), against the oracle at
   1e-12 relative L2 (the forced stage kernels run in the 384^2 L-shape
   configuration test, also above the threshold);
+* the same on meshes whose elements start their corner lists anywhere, so the
+  traces that streaming stages read from the LDS tile of their own workgroup
+  run along the neighbour's side in either direction;
 * one WaveHoltz fixed-point update (the filter-accumulating stage kernels)
   on a mesh above the threshold: bitwise equal under every schedule."""
 from __future__ import annotations
@@ -62,6 +65,37 @@ def test_streaming_rk4_matches_oracle_under_every_schedule(cuda, n, nx, leg):
         err = rel_l2(du.cpu().numpy(), ref)
         print(f"  schedule {k} ({gw.schedule()[1]} threads): rel L2 {err:.3e}", flush=True)
         assert err < TOL64
+        del gw, du
+
+
+@pytest.mark.parametrize("n,nx,leg,precision", [(4, 512, False, capi.F64), (9, 220, False, capi.F64),
+                                                (7, 280, True, capi.F64), (6, 470, False, capi.F32),
+                                                (9, 310, True, capi.F32)])
+def test_streaming_rotated_elements_match_oracle(cuda, n, nx, leg, precision):
+    """Elements whose corner lists start at any corner.  FP64 at 1e-12.  FP32
+    at 1e-6: the state's rounding and the ten stages' stochastic ones, 2^-23 at
+    most each and in random directions, stay below 2^-23 sqrt(11) = 4e-7."""
+    torch = cuda
+    v, e = meshgen.perturbed_rect(nx, nx, 0.2, 930 + n)
+    turn = np.random.RandomState(n).randint(0, 4, len(e))
+    e = np.ascontiguousarray(np.asarray(e)[np.arange(len(e))[:, None], (np.arange(4) + turn[:, None]) % 4])
+    gm, om = capi.Mesh(v, e), O.Mesh(v, e)
+    bc = (np.arange(gm.n_boundary) % 3).astype(np.int32)
+    rsz, tol = (4, 1e-6) if precision == capi.F32 else (8, TOL64)
+    assert 3 * (3 * n * n * gm.n_elem) * rsz > CACHE
+    print(f"streaming, rotated elements: {nx}^2, n={n}, legendre={leg}, {8 * rsz} bits", flush=True)
+    u0 = _state(gm, n)
+    dt = 0.5 * gm.min_h() / n**2
+    ref, _ = O.Wave(om, n, bc, legendre=leg).rk4(u0, dt, 2)
+    for k in range(capi.schedule_count()[0]):
+        gw = capi.Wave2D(gm, n, bc, precision=precision, basis=capi.GAUSS_LEGENDRE if leg else capi.GAUSS_LOBATTO)
+        gw.set_schedule(k)
+        du = torch.tensor(u0, dtype=gw.torch_dtype, device="cuda")
+        gw.rk4(du, dt, 2)
+        torch.cuda.synchronize()
+        err = rel_l2(du.cpu().numpy(), ref)
+        print(f"  schedule {k} ({gw.schedule()[1]} threads): rel L2 {err:.3e}", flush=True)
+        assert err < tol
         del gw, du
 
 
