@@ -1896,7 +1896,10 @@ void launch_conv(const wdg_cnn_s& n, hipStream_t s, const uint16_t* in, int in_l
                 // at 128^2 x 16 images 512 pixels per tile on level 0 (32 -> 32
                 // channels 12.7 us, 17.4 us with 256 of four waves), 256, 128
                 // and 64 on levels 1, 2 and 3 (256 -> 256 channels of level 3
-                // 13.5 us, 17.0 us with 256 pixels)
+                // 13.5 us, 17.0 us with 256 pixels).  Small batches gain too:
+                // a training step against conv3_k32_kernel and wgrad3_tr_kernel
+                // at every width, 128^2 x 1, 5 and 16 images 687 -> 574, 941 ->
+                // 737 and 1404 -> 1099 us, 64^2 594 -> 549, 721 -> 591, 838 -> 714
                 const int WX = std::min(W, 64) / 16, cob = cout / 32;
                 auto blocks = [&](int r, int nw) { return (long long)npix / (16 * r * nw) * cob; };
                 auto fits = [&](int r, int nw) { return r * nw / WX <= H && blocks(r, nw) >= 512; };
