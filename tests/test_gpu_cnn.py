@@ -143,6 +143,26 @@ def test_dg_image_maps(cuda):
     assert float(torch.linalg.norm(W2 - W) / torch.linalg.norm(W)) < 1e-7
 
 
+def test_features_round_through_float(cuda):
+    """A feature is the bf16 of the float of its double (as the oracle rounds).
+    At a source's own node the forcing is gain * amp: a double just above the
+    float that lies halfway between two bf16 values goes to the even one, and
+    so does one just below it."""
+    torch = cuda
+    M, n, ld = 2, 3, 16
+    mesh = capi.Mesh.uniform_rect(M, 0.0, 1.0, M, 0.0, 1.0)
+    nodes = mesh.nodes(n)
+    nd = torch.tensor(nodes.reshape(-1), device="cuda")
+    x0, y0 = np.asarray(nodes).reshape(-1, 2)[0]
+    sd = torch.tensor([x0, y0, 0.05, 1.0], dtype=torch.float64, device="cuda")
+    xd = torch.empty((M * M, ld), dtype=torch.bfloat16, device="cuda")
+    for half, even in ((1.0 + 2.0 ** -8, 1.0), (1.0 + 3 * 2.0 ** -8, 1.0 + 2.0 ** -6)):
+        for off in (-(2.0 ** -40), 0.0, 2.0 ** -40):
+            capi.ws_features(nd, n, M * M, sd, 1, half + off, 0.0, 0.0, 0.0, (0.0, 0.0, 1.0, 1.0), ld, xd)
+            torch.cuda.synchronize()
+            assert float(xd[0, 0]) == even, (half, off)
+
+
 @pytest.mark.parametrize("M,B", [(128, 16), (32, 128), (32, 256)])
 def test_convolution_tiles_agree(cuda, M, B):
     """Tiles of conv3_row_kernel against its smallest, which one image alone

@@ -1625,11 +1625,21 @@ __device__ __forceinline__ void bessel_j0_y0(double x, double& j0, double& y0)
 // 1-4 sources, 18 us here.
 constexpr int kFeatSrc = 32;  // sources staged at a time
 
+// bf16 of a double through its float, as the oracle rounds: the compiler would
+// otherwise convert in one step, which differs where the float is halfway
+// between two bf16 values.
+__device__ __forceinline__ uint16_t d2bf(double d)
+{
+    float f = (float)d;
+    asm("" : "+v"(f));
+    return f2bf(f);
+}
+
 __global__ __launch_bounds__(256) void features_kernel(const double* nodes, int nn, int nel, const double* src, int ns,
                                                        double gain, double omega, float omega_feat, double green_gain,
                                                        double x0, double y0, double x1, double y1, uint16_t* x, int ld)
 {
-    __shared__ double s_src[kFeatSrc][6];  // x, y, 2 sigma^2, sigma^2, amp, m
+    __shared__ double s_src[kFeatSrc][6];  // x, y, 2 sigma^2, sigma, amp, m
     const bool green = green_gain != 0.0;
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = q < (long long)nel * nn;
@@ -1647,7 +1657,7 @@ __global__ __launch_bounds__(256) void features_kernel(const double* nodes, int 
             o[0] = p[0];
             o[1] = p[1];
             o[2] = 2.0 * sg * sg;
-            o[3] = sg * sg;
+            o[3] = sg;
             o[4] = amp;
             o[5] = amp * 6.283185307179586 * sg * sg * exp(-0.5 * omega * omega * sg * sg);
         }
@@ -1656,10 +1666,11 @@ __global__ __launch_bounds__(256) void features_kernel(const double* nodes, int 
         for (int c = 0; c < nc; ++c) {
             const double* p = s_src[c];
             const double dx = px - p[0], dy = py - p[1], r2 = dx * dx + dy * dy;
-            f += p[4] * exp(-r2 / p[2]);
-            if (green) {
-                double jv, yv;
-                bessel_j0_y0(omega * sqrt(r2 + p[3]), jv, yv);
+            double jv = 0.0, yv = 0.0;
+            if (green) bessel_j0_y0(omega * sqrt(r2 + p[3] * p[3]), jv, yv);
+            {
+#pragma clang fp contract(off)  // each source's term is rounded before it is added
+                f += p[4] * exp(-r2 / p[2]);
                 gj += p[5] * jv;
                 gy += p[5] * yv;
             }
@@ -1667,14 +1678,14 @@ __global__ __launch_bounds__(256) void features_kernel(const double* nodes, int 
     }
     if (!active) return;
     uint16_t* const xe = x + (size_t)e * ld;
-    xe[k] = f2bf((float)(gain * f));
+    xe[k] = d2bf(gain * f);
     if (green) {
-        xe[nn + k] = f2bf((float)(green_gain * gj));
-        xe[2 * nn + k] = f2bf((float)(green_gain * gy));
+        xe[nn + k] = d2bf(green_gain * gj);
+        xe[2 * nn + k] = d2bf(green_gain * gy);
     }
     const int base = green ? 3 * nn : nn;
     for (int c = base + k; c < ld; c += nn) {
-        float v = 0.f;
+        double v = 0.0;
         if (c == base) {
             v = omega_feat;
         } else if (c == base + 1 || c == base + 2) {
@@ -1683,9 +1694,9 @@ __global__ __launch_bounds__(256) void features_kernel(const double* nodes, int 
             for (int i = 0; i < nn; ++i) m += el[2 * i + d];
             m /= nn;
             const double lo = d ? y0 : x0, hi = d ? y1 : x1;
-            v = (float)(2.0 * (m - lo) / (hi - lo) - 1.0);
+            v = 2.0 * (m - lo) / (hi - lo) - 1.0;
         }
-        xe[c] = f2bf(v);
+        xe[c] = d2bf(v);
     }
 }
 
