@@ -215,6 +215,18 @@ def test_weight_gradient_of_an_odd_number_of_strips(cuda, M, base, B):
         assert err < 1e-5, name  # below 2^-24 * 2^7, as above
 
 
+@pytest.mark.parametrize("M,B,want", [(32, 2, 1.6441795826), (64, 1, 1.74118685722), (128, 2, 1.79015147686)])
+def test_convolution_sums_in_tap_order(cuda, M, B, want):
+    """Outputs add their slices and taps in one order at every width, that of
+    conv3_k32_kernel, so a network's outputs do not move with the kernel that
+    a layer takes.  The losses are those of a build that ran that kernel at
+    every width; another order puts some values on the other side of a bf16
+    boundary and moves them by 3e-7 to 4e-5, against the 11 digits given."""
+    net, p, x, t, xd, td = _setup(cuda, M=M, base=32, in_ld=48, B=B, seed=9)
+    loss, _ = net.loss_grad(xd, td)
+    assert loss == pytest.approx(want, rel=2e-10)
+
+
 def test_row_convolution_matches_oracle(cuda):
     """conv3_row_kernel at widths 32 and 16 (conv3_k32_kernel at 8 and 4), with
     a last slice of 16 input channels, against the oracle."""

@@ -438,10 +438,14 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
 // 3x3 convolution of images at least 16 pixels wide, with the operands of
 // conv3_k32_kernel.  A wave there reads one pixel fragment from LDS per tap
 // for TA MFMAs, and its LDS reads took 1.5-2.3 times the MFMAs' cycles.  Here
-// a wave owns R rows of 16 pixels x 32 output channels and walks the R + 2
-// input rows once per horizontal tap: each fragment it reads feeds the MFMAs
-// of all three vertical taps, so a 32-channel slice costs 18 + 3 (R + 2)
-// fragment reads for 18 R MFMAs.  NW waves cover TW = min(W, 64) x TH pixels;
+// a wave owns R rows of 16 pixels x 32 output channels and keeps the fragments
+// of R input rows at the three horizontal taps in registers; the next vertical
+// tap reads one row more.  Each fragment so feeds the MFMAs of all three
+// vertical taps, and a 32-channel slice costs 18 + 3 (R + 2) fragment reads for
+// 18 R MFMAs.  Every output adds its slices and taps in conv3_k32_kernel's
+// order, so the widths give the same sums (with the taps of a column first,
+// predictions moved by 3e-3 through bf16 boundaries, at the same speed).
+// NW waves cover TW = min(W, 64) x TH pixels;
 // the tile's halo and the slice's weights go from global memory straight to
 // LDS (16 bytes per lane, no registers), halo pixels outside the image and
 // channels past the last read as zeros past
@@ -532,30 +536,29 @@ __global__ __launch_bounds__(64 * NW) void conv3_row_kernel(ConvArgs a)
         for (int k = 0; k < T::NWP; ++k) load_to_lds16(rw, woff[k], 2u * c0, s_w + 8 * (NTHR * k + 64 * wave));
         __builtin_amdgcn_s_waitcnt(0);  // the loads to LDS have landed
         __syncthreads();
+        const uint16_t* const src = s_in + (wy * R * HW2 + 16 * wx + ln) * 32 + 8 * kq;
+        bf16x8 bv[R + 2][3];
 #pragma unroll
-        for (int hx = 0; hx < 3; ++hx) {
-            bf16x8 av[3][TA];
+        for (int hy = 0; hy < 3; ++hy)
 #pragma unroll
-            for (int hy = 0; hy < 3; ++hy)
+            for (int hx = 0; hx < 3; ++hx) {
+                bf16x8 av[TA];
 #pragma unroll
                 for (int i = 0; i < TA; ++i)
-                    av[hy][i] = __builtin_bit_cast(
+                    av[i] = __builtin_bit_cast(
                         bf16x8, *reinterpret_cast<const uint4*>(
                                     s_w + ((3 * hy + hx) * CO_T + 16 * i + ln) * 32 + 8 * kq));
-            const uint16_t* src = s_in + (wy * R * HW2 + 16 * wx + ln + hx) * 32 + 8 * kq;
 #pragma unroll
-            for (int r = 0; r < R + 2; ++r) {
-                const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + r * HW2 * 32));
-#pragma unroll
-                for (int hy = 0; hy < 3; ++hy) {
-                    if (r - hy < 0 || r - hy >= R) continue;
+                for (int o = 0; o < R; ++o) {
+                    const int r = o + hy;
+                    if (hy == 0 || o == R - 1)  // the other rows were read for the tap above
+                        bv[r][hx] =
+                            __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + (r * HW2 + hx) * 32));
 #pragma unroll
                     for (int i = 0; i < TA; ++i)
-                        acc[i][r - hy] =
-                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[hy][i], bv, acc[i][r - hy], 0, 0, 0);
+                        acc[i][o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[r][hx], acc[i][o], 0, 0, 0);
                 }
             }
-        }
     }
 #pragma unroll
     for (int i = 0; i < TA; ++i) {
