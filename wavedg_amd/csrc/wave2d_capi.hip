@@ -3,6 +3,7 @@
 // bookkeeping, precision conversion).
 #include "../../include/wavedg_hip.h"
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -888,6 +889,7 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
         if (m.min_corner_detj() <= 0.0) fail(WDG_ERR_MESH, "mesh has an inverted or degenerate element (det J <= 0)");
         wdg::FaceTables ft;
         std::string err;
+        ft.info.reserve(4 * (size_t)m.n_elem() + 2 * (size_t)m.n_boundary());  // room for the boundary lists
         if (!m.face_tables(bc, ft, err)) fail(WDG_ERR_INVALID, err);
         hip_check(hipGetDevice(&op->dev), "hipGetDevice");
         op->n = n_colloc;
@@ -938,17 +940,16 @@ static int create_collocated(wdg_mesh mesh, int n_colloc, int basis_type, const 
         // the elements with a boundary side, then the workgroups of the collocated
         // kernels that hold one, ride behind the info words in one array
         {
+            std::vector<int32_t> bel(m.n_boundary()), blk;
+            for (int k = 0; k < m.n_boundary(); ++k) bel[k] = m.edge(k, false).el[0];
+            std::sort(bel.begin(), bel.end());
+            bel.erase(std::unique(bel.begin(), bel.end()), bel.end());
             const int epb = wdg::elems_per_block(n);
-            std::vector<int32_t> blk;
-            const size_t ni = ft.info.size();
-            for (int e = 0; e < op->nel; ++e) {
-                const int32_t* nb = &ft.nbr[4 * (size_t)e];
-                if ((nb[0] | nb[1] | nb[2] | nb[3]) >= 0) continue;  // no side is -1
-                ft.info.push_back(e);
+            for (int e : bel)
                 if (blk.empty() || blk.back() != e / epb) blk.push_back(e / epb);
-            }
-            op->n_bel = (int)(ft.info.size() - ni);
+            op->n_bel = (int)bel.size();
             op->n_bblk = (int)blk.size();
+            ft.info.insert(ft.info.end(), bel.begin(), bel.end());
             ft.info.insert(ft.info.end(), blk.begin(), blk.end());
         }
         op->d_info = static_cast<int32_t*>(dmalloc(sizeof(int32_t) * ft.info.size()));
