@@ -3,9 +3,9 @@
 // bookkeeping, precision conversion).
 #include "../../include/wavedg_hip.h"
 
-#include <algorithm>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
