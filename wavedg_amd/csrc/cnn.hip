@@ -448,10 +448,9 @@ __global__ __launch_bounds__(256) void conv3_k32_kernel(ConvArgs a)
 // NW waves cover TW = min(W, 64) x TH pixels;
 // the tile's halo and the slice's weights go from global memory straight to
 // LDS (16 bytes per lane, no registers), halo pixels outside the image and
-// channels past the last read as zeros past
-// the buffer's end.  What bounds it now is the latency
-// of one slice's loads and the two or three workgroups a CU holds to cover
-// it.  128^2 x 16 images, forward / backward-data of all 3x3 layers: 270 /
+// channels past the last read as zeros past the buffer's end.  What bounds it
+// now is the latency of one slice's loads and the two or three workgroups a CU
+// holds to cover it.  128^2 x 16 images, forward / backward-data of all 3x3 layers: 270 /
 // 297 us with conv3_k32_kernel at every width, 182 / 182 us here (192 / 192
 // with per-part pointers and a run-time tile width); blocks of 64 output
 // channels measured slower at every level (fewer workgroups).
@@ -844,7 +843,11 @@ __global__ __launch_bounds__(64 * kWgWaves) void wgrad3_tr_kernel(WgradArgs a)
 // gradients and reductions of all 3x3 layers: 422 us with wgrad3_tr_kernel,
 // 337 here.  What bounds it now is the latency of a tile's loads with one tile
 // in flight per CU.
-constexpr int kWgRowTarget = 256;  // workgroups a layer aims for: one per CU
+// Workgroups a layer aims for: one per CU.  The shorter tiles fit twice, but 512
+// of them add partial rows to write and reduce: a training step of 8 images at
+// 64^2 470 -> 479 us, 2 at 128^2 448 -> 454, 1 and 16 at 64^2 and 1, 4 and 8
+// at 128^2 within 0.3 %.
+constexpr int kWgRowTarget = 256;
 
 // TW = 32, or 16 on 16-pixel images (two strips per tile)
 template <int RW, int TW>
