@@ -609,8 +609,15 @@ __global__ __launch_bounds__((Shape<N, TGT>::NT), (sizeof(R) == 4 ? WDG_MIN_WAVE
     // those along a row of elements) from LDS: fewer cache requests beside the
     // streams (512^2 P = 7 FP64 299 -> 279 us, 701 x 499 P = 5 FP32 129 -> 121,
     // 301 x 257 P = 6 Gauss-Legendre 107 -> 101).  Stages that fit the cache are
-    // 0-4 % slower with it (the longer way from the barrier to the fluxes).
-    constexpr bool INB = NT;
+    // 0-4 % slower with it (the longer way from the barrier to the fluxes).  So are
+    // the streaming Gauss-Legendre stages of a few orders, whose lanes read N
+    // values a trace: P = 7 (50M unknowns, from memory and from LDS: FP32 215 and
+    // 219 us, 162 and 167 on a 1:2 grid; FP64 447 and 448, 334 and 337), FP32 P = 8
+    // (241 and 247, 183 and 191) and FP64 P = 2 (346 and 350, 256 and 262).  The
+    // other Gauss-Legendre orders gain 0-12 % (FP64 P = 4 405 -> 361), Gauss-Lobatto
+    // ones 0-9 %.
+    constexpr bool SLOW_INB = LEG && (N == 8 || (sizeof(R) == 4 ? N == 9 : N == 3));
+    constexpr bool INB = NT && !SLOW_INB;
     using L = OpLds<N, R, VOL, IFACE || BFACE, TGT, LEG>;
     __shared__ __align__(16) unsigned char lds[L::bytes];
 
