@@ -118,7 +118,7 @@ def test_third_buffer_stays_below_a_sixteenth_of_the_free_memory(cuda):
     size = 8 * w.ndof
     x = torch.zeros(w.ndof, dtype=torch.float64, device="cuda")
     w.rk4(x, dt, 2)
-    hold = []  # leave about eight states free, in pieces the box can give
+    hold = []  # leave about eight states free
     while (left := _free(torch) - 8 * size) > (1 << 28):
         hold.append(torch.empty(min(left, 16 << 30), dtype=torch.uint8, device="cuda"))
     free = _free(torch)
