@@ -143,6 +143,27 @@ def test_dg_image_maps(cuda):
     assert float(torch.linalg.norm(W2 - W) / torch.linalg.norm(W)) < 1e-7
 
 
+@pytest.mark.parametrize("ns", [0, 1, 32, 33, 70])
+def test_features_of_many_sources(cuda, ns):
+    """Sources are staged 32 at a time, also by the idle threads of the last
+    workgroup (35 elements of 9 nodes are 315 threads)."""
+    torch = cuda
+    n, ld = 3, 32
+    mesh = capi.Mesh.uniform_rect(7, 0.0, 1.0, 5, 0.0, 1.0)
+    nodes = mesh.nodes(n)
+    r = np.random.default_rng(ns)
+    src = np.column_stack([r.uniform(0.0, 1.0, (ns, 2)), r.uniform(0.05, 0.3, ns), r.uniform(0.5, 1.5, ns)])
+    sd = torch.tensor(src.reshape(-1), device="cuda")
+    xd = torch.full((35, ld), 5.0, dtype=torch.bfloat16, device="cuda")
+    box = (0.0, 0.0, 1.0, 1.0)
+    capi.ws_features(torch.tensor(nodes.reshape(-1), device="cuda"), n, 35, sd, ns, 0.7, 9.0, 0.5, 0.3, box, ld, xd)
+    torch.cuda.synchronize()
+    got = xd.float().cpu().numpy().astype(np.float64)
+    want = co.bf16(co.features(nodes, n, src, 0.7, 0.5, box, ld, omega=9.0, green_gain=0.3))
+    # one bf16 step where the Bessel polynomials (1e-7 each) round differently
+    assert np.all(np.abs(got - want) <= 2.0 ** -7 * np.abs(want) + 1e-6)
+
+
 def test_features_round_through_float(cuda):
     """A feature is the bf16 of the float of its double (as the oracle rounds).
     At a source's own node the forcing is gain * amp: a double just above the
